@@ -5,12 +5,31 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <string>
 #include <vector>
 
 #include "../../include/goneuron_hip.h"
 
 namespace gn {
+
+// hipFuncSetAttribute(MaxDynamicSharedMemorySize) holds per device and per
+// kernel.  set[d] is the largest size already set on device d for one kernel:
+// a later launch that needs more LDS (a larger H) sets it again.
+constexpr int kAttrDevices = 64;
+inline hipError_t ensure_lds_attr(const void *fn, int bytes, std::atomic<int> (&set)[kAttrDevices]) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= kAttrDevices) return hipErrorInvalidDevice;
+  if (set[dev].load(std::memory_order_relaxed) >= bytes) return hipSuccess;
+  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return e;
+  int cur = set[dev].load(std::memory_order_relaxed);
+  while (cur < bytes && !set[dev].compare_exchange_weak(cur, bytes)) {
+  }
+  return hipSuccess;
+}
 
 // Activation derivative kinds used by kernels.  Computed from the saved
 // *output* of the layer: out = act(pre) is deterministic, so relu'(pre) ==
@@ -292,6 +311,62 @@ hipError_t launch_bn_bwd_eval(const float *g, const float *gb, const float *rv, 
 hipError_t launch_avgpool_fwd(const float *x, float *out, const PoolShape &s, int B, hipStream_t st);
 hipError_t launch_avgpool_bwd(const float *gout, float *gin, const PoolShape &s, int B, hipStream_t st);
 
+// exp(t) in float64 for a float32 result: t = n ln 2 + r with |r| <= ln 2 / 2
+// and the Taylor polynomial of degree 9 (its remainder r^10 / 10! is below
+// 7e-12 of the result, so the float32 rounding is the float64 value's but for
+// one tie in 4,000).  A third of the instructions and registers of the
+// library's exp, which answers to 1e-16.  |t| <= 700; NaN in, NaN out.
+__device__ __forceinline__ double exp_r10(double t, double &n) {
+  n = __builtin_rint(t * 1.4426950408889634);
+  return __builtin_fma(n, -0.6931471805599453, t);
+}
+// (exp(r) - 1) / r
+__device__ __forceinline__ double expm1_poly(double r) {
+  double p = 1.0 / 3628800.0;
+  p = __builtin_fma(p, r, 1.0 / 362880.0);
+  p = __builtin_fma(p, r, 1.0 / 40320.0);
+  p = __builtin_fma(p, r, 1.0 / 5040.0);
+  p = __builtin_fma(p, r, 1.0 / 720.0);
+  p = __builtin_fma(p, r, 1.0 / 120.0);
+  p = __builtin_fma(p, r, 1.0 / 24.0);
+  p = __builtin_fma(p, r, 1.0 / 6.0);
+  p = __builtin_fma(p, r, 0.5);
+  return __builtin_fma(p, r, 1.0);
+}
+// 1 / (1 + float32(exp(-x))), the reference's float32 expression around a
+// float64 exp (the clamp keeps the exponent in range: exp(100) is already
+// infinite and exp(-100) lost beside 1 in float32)
+__device__ __forceinline__ float sigmoid_f64(float x) {
+  const float c = x > 100.0f ? 100.0f : x < -100.0f ? -100.0f : x;
+  double n;
+  const double r = exp_r10(-(double)c, n);
+  const double e = __builtin_ldexp(__builtin_fma(expm1_poly(r), r, 1.0), (int)n);
+  return 1.0f / (1.0f + (float)e);
+}
+// float32(tanh(x)) as (e^2x - 1) / (e^2x + 1) in float64, the numerator from
+// exp - 1 of the reduced argument so that small x keep their relative
+// precision; float64 tanh rounds to 1 in float32 well before |x| = 20.
+__device__ __forceinline__ float tanh_f64(float x) {
+  const float c = x > 20.0f ? 20.0f : x < -20.0f ? -20.0f : x;
+  double n;
+  const double r = exp_r10(2.0 * (double)c, n);
+  const double s = __builtin_ldexp(1.0, (int)n);
+  const double m = __builtin_fma(s, expm1_poly(r) * r, s - 1.0), d = m + 2.0;
+  double y = __builtin_amdgcn_rcp(d);
+  y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+  return (float)(m * y);
+}
+
+// A workgroup barrier for data passed through LDS: waits for this wave's LDS
+// operations only.  __syncthreads also waits for every outstanding global
+// load and store of the wave, which puts a memory round trip into each step
+// of a recurrence that stores its state or prefetches the next step's inputs;
+// no thread may rely on it to see another's global writes.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ---- the reference's LCG (layer.go:61-81) on the device ----
 constexpr uint64_t LCG_A = 6364136223846793005ull, LCG_C = 1ull;
 // state after n steps of s -> a s + c (binary powers of the affine map)
@@ -329,10 +404,11 @@ hipError_t launch_moe_backward_deltas(const float *g, const float *eout, const f
 
 // ---- SequenceUnroller(GRU) ----
 bool gru_supported(int H);
+// act: the gates' activations u, r, c of every step, [B*T][3H].
 // seq (returnSequences): out [B][T][H]; g dL/dh_t [B][T][H] (else [B][H])
-hipError_t launch_gru_fwd(const float *xw, const float *WhT, float *pre, float *hprev, float *rh,
+hipError_t launch_gru_fwd(const float *xw, const float *WhT, float *act, float *hprev, float *rh,
                           float *out, int B, int T, int H, hipStream_t s, int seq = 0);
-hipError_t launch_gru_bwd(const float *g, const float *pre, const float *hprev, const float *Wh,
+hipError_t launch_gru_bwd(const float *g, const float *act, const float *hprev, const float *Wh,
                           float *dG, int B, int T, int H, hipStream_t s, int seq = 0);
 
 // ---- SequenceUnroller(LSTM) ----

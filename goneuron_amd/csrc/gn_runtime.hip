@@ -545,7 +545,7 @@ struct LayerRT {
   // partial sums [2][maxB*C], running mean / var [C]
   int C = 0, HW = 0;
   float *bnst = nullptr, *bnpart = nullptr, *rmean = nullptr, *rvar = nullptr;
-  // SequenceUnroller(GRU): pre-activations [B*T][3H], h before each step and
+  // SequenceUnroller(GRU): gate activations [B*T][3H], h before each step and
   // r * h_prev [B*T][H] (xw, WhT, Dg, S as for the LSTM, sized for 3 gates)
   float *gpre = nullptr, *ghprev = nullptr, *grh = nullptr;
   // MoE: E experts, top K; gate logits / probabilities / deltas [B][E], routes

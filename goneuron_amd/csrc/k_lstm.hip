@@ -22,27 +22,7 @@
 // dWh = (w dG)^T hPrev, db = sum w dG.
 #include "gn_common.h"
 
-#include <atomic>
-
 namespace gn {
-
-// hipFuncSetAttribute(MaxDynamicSharedMemorySize) holds per device and per
-// kernel.  set[d] is the largest size already set on device d for one kernel:
-// a later launch that needs more LDS (a larger H) sets it again.
-static constexpr int kAttrDevices = 64;
-static hipError_t ensure_lds_attr(const void *fn, int bytes, std::atomic<int> (&set)[kAttrDevices]) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= kAttrDevices) return hipErrorInvalidDevice;
-  if (set[dev].load(std::memory_order_relaxed) >= bytes) return hipSuccess;
-  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) return e;
-  int cur = set[dev].load(std::memory_order_relaxed);
-  while (cur < bytes && !set[dev].compare_exchange_weak(cur, bytes)) {
-  }
-  return hipSuccess;
-}
 
 __device__ __forceinline__ float sigm(float x) { return 1.0f / (1.0f + (float)exp((double)(-x))); }
 __device__ __forceinline__ float tanh32(float x) { return (float)tanh((double)x); }
