@@ -561,15 +561,17 @@ hipError_t launch_rms_fwd(const float *x, const float *gam, float *y, float *rms
 hipError_t launch_rms_bwd(const float *g, const float *x, const float *gam, const float *rms,
                           float *dx, float *gx, int rows, int N, hipStream_t s);
 bool attn_supported(int T, int D, int NH);  // the fused kernels: T <= 128, D / NH <= 32
-// Attention of any T and head size through batched GEMMs over the (sample,
-// head) pairs and row kernels: the scores / probabilities and their
-// gradients are materialised in `S` (attn_gemm_floats(B, T, NH) floats)
-size_t attn_gemm_floats(int B, int T, int NH);
-hipError_t launch_attn_fwd_gemm(const float *Q, const float *K, const float *V, float *O, int B, int T,
-                                int D, int NH, int causal, float *S, hipStream_t s);
-hipError_t launch_attn_bwd_gemm(const float *Q, const float *K, const float *V, const float *GO,
-                                float *GQ, float *GK, float *GV, int B, int T, int D, int NH, int causal,
-                                float *S, hipStream_t s);
+// Attention of any T and head size: heads of up to 128 in kernels that stage
+// the other side's rows, wider ones through batched GEMMs over the (sample,
+// head) pairs and row kernels.  `S` (attn_work_floats) carries what the
+// forward leaves for the backward: (maximum, 1 / sum) per row, or the
+// materialised scores and their gradients.  O: the forward's output.
+size_t attn_work_floats(int B, int T, int D, int NH);
+hipError_t launch_attn_fwd_any(const float *Q, const float *K, const float *V, float *O, int B, int T,
+                               int D, int NH, int causal, float *S, hipStream_t s);
+hipError_t launch_attn_bwd_any(const float *Q, const float *K, const float *V, const float *O, const float *GO,
+                               float *GQ, float *GK, float *GV, int B, int T, int D, int NH, int causal,
+                               float *S, hipStream_t s);
 hipError_t launch_attn_fwd(const float *Q, const float *K, const float *V, float *O, int B, int T,
                            int D, int NH, int causal, hipStream_t s);
 // TS (may be null): the per-sample token sums of gQ, gK, gV ([B][D] each, member m at TS + m * tss)

@@ -264,7 +264,7 @@ MhaBufs mha_carve(float *w, int B, int T, int D, int NH, int rope, size_t *float
   const size_t half = (size_t)std::max(D / std::max(NH, 1) / 2, 1);
   m.rcos = rope ? cv.take((size_t)T * half) : nullptr;
   m.rsin = rope ? cv.take((size_t)T * half) : nullptr;
-  m.SC = attn_supported(T, D, NH) ? nullptr : cv.take(attn_gemm_floats(B, T, NH));
+  m.SC = attn_supported(T, D, NH) ? nullptr : cv.take(attn_work_floats(B, T, D, NH));
   if (floats) *floats = cv.off;
   return m;
 }
@@ -316,7 +316,7 @@ int mha_forward_impl(gn_ctx *c, const float *x, const float *params, float *out,
   {
     KTimer kt(c, GN_KCLASS_OTHER, "attn_fwd", attn_flops(B, T, NH, hd, causal, false));
     if (m.SC)
-      HIP_OK(c, launch_attn_fwd_gemm(m.Q, m.K, m.V, m.O, B, T, D, NH, causal, m.SC, c->stream));
+      HIP_OK(c, launch_attn_fwd_any(m.Q, m.K, m.V, m.O, B, T, D, NH, causal, m.SC, c->stream));
     else
       HIP_OK(c, launch_attn_fwd(m.Q, m.K, m.V, m.O, B, T, D, NH, causal, c->stream));
   }
@@ -369,7 +369,7 @@ int mha_backward_impl(gn_ctx *c, const float *x, const float *params, const floa
   {
     KTimer kt(c, GN_KCLASS_OTHER, "attn_bwd", attn_flops(B, T, NH, hd, causal, true));
     if (m.SC)
-      HIP_OK(c, launch_attn_bwd_gemm(m.Q, m.K, m.V, m.GO, m.GQ, m.GK, m.GV, B, T, D, NH, causal, m.SC,
+      HIP_OK(c, launch_attn_bwd_any(m.Q, m.K, m.V, m.O, m.GO, m.GQ, m.GK, m.GV, B, T, D, NH, causal, m.SC,
                                      c->stream));
     else
       HIP_OK(c, launch_attn_bwd(m.Q, m.K, m.V, m.GO, m.GQ, m.GK, m.GV, B, T, D, NH, causal, c->stream));

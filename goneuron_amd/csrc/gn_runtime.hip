@@ -887,7 +887,7 @@ static int alloc_batch(gn_model *M) {
         if ((rc = model_balloc(M, nb * D, &t.TS2))) return rc;
       }
       if (!attn_supported(R.T, R.D, R.NH) &&
-          (rc = model_balloc(M, attn_gemm_floats(max_batch, R.T, R.NH), &t.SC)))
+          (rc = model_balloc(M, attn_work_floats(max_batch, R.T, R.D, R.NH), &t.SC)))
         return rc;
       if (R.d.block_act == GN_BLOCK_ACT_SWIGLU) {
         if ((rc = model_balloc(M, rows * 2 * FF, &t.Z))) return rc;
@@ -1006,7 +1006,7 @@ static int alloc_batch(gn_model *M) {
         if ((rc = model_balloc(M, nb * D, &t.TS2))) return rc;
       }
       if (!attn_supported(R.T, R.D, R.NH) &&
-          (rc = model_balloc(M, attn_gemm_floats(max_batch, R.T, R.NH), &t.SC)))
+          (rc = model_balloc(M, attn_work_floats(max_batch, R.T, R.D, R.NH), &t.SC)))
         return rc;
     }
     if (R.d.kind == GN_LAYER_MAXPOOL2D) {
@@ -1703,7 +1703,7 @@ static int tb_forward(gn_model *M, LayerRT &R, const float *X, int B, float *cls
   {
     KTimer kt(c, GN_KCLASS_OTHER, "attn_fwd", attn_flops(B, R.T, R.NH, D / R.NH, R.causal, false));
     if (t.SC)
-      HIP_OK(c, launch_attn_fwd_gemm(t.Q, t.K, t.V, t.O, B, R.T, D, R.NH, R.causal, t.SC, c->stream));
+      HIP_OK(c, launch_attn_fwd_any(t.Q, t.K, t.V, t.O, B, R.T, D, R.NH, R.causal, t.SC, c->stream));
     else
       HIP_OK(c, launch_attn_fwd(t.Q, t.K, t.V, t.O, B, R.T, D, R.NH, R.causal, c->stream));
   }
@@ -1878,7 +1878,7 @@ static int tb_backward(gn_model *M, LayerRT &R, const float *X, float *gin, int 
   {
     KTimer kt(c, GN_KCLASS_OTHER, "attn_bwd", attn_flops(B, T, R.NH, D / R.NH, R.causal, true));
     if (t.SC)
-      HIP_OK(c, launch_attn_bwd_gemm(t.Q, t.K, t.V, t.GO, t.GQ, t.GK, t.GV, B, T, D, R.NH, R.causal, t.SC,
+      HIP_OK(c, launch_attn_bwd_any(t.Q, t.K, t.V, t.O, t.GO, t.GQ, t.GK, t.GV, B, T, D, R.NH, R.causal, t.SC,
                                      c->stream));
     else
       HIP_OK(c, launch_attn_bwd(t.Q, t.K, t.V, t.GO, t.GQ, t.GK, t.GV, B, T, D, R.NH, R.causal, c->stream,

@@ -1553,8 +1553,520 @@ bool attn_supported(int T, int D, int NH) {
 }
 
 // ---------------------------------------------------------------------------
-// Attention of any sequence length and head size (the fused kernels above
-// hold T <= 128 keys and 32-wide heads in LDS).  The scores of every (sample,
+// Attention of any sequence length with heads of up to 128 (what the kernels
+// above do not hold in LDS at once), on fp32 MFMA 16x16x4 with their operand
+// layouts and the same mask convention (key tiles that lie wholly above the
+// diagonal contribute exact zeros).  Nothing of size T x T is written: the
+// forward keeps a running row maximum and sum over stages of keys and leaves
+// (maximum, 1 / sum) per row for the backward, which recomputes the
+// probabilities.  A workgroup is four waves that share the staged rows of the
+// other side in LDS.
+// The materialised form (batched GEMMs over the pairs, below) took a launch
+// per (sample, head) pair when T is odd, and otherwise moved 2 T^2 floats per
+// pair through HBM seven times.  The whole layer, forward + backward: B 8, T
+// 197, 3 heads of 64 1207 -> 106 us; B 4, T 512, 8 heads of 64, causal 310 ->
+// 216; a GPT step at B 16, T 256, 8 heads of 32 510 -> 319.  What bounds them
+// is the matrix pipe (forward 17 of 27 kilocycles at B 4, T 512, backward 62)
+// and, beside it, the vector work of the exponentials and the staging.
+// ---------------------------------------------------------------------------
+constexpr int FA_B = 64;    // rows per workgroup (16 per wave) where they fill the chip
+constexpr int FA_NT = 256;
+
+// exp of a float32 argument <= 0 in float32: x = n ln 2 + r with n ln2_hi
+// exact, the Taylor polynomial of degree 7 in |r| <= ln 2 / 2 and one rounding
+// at the end: 1.03 ulp at most, 0.31 rms (float64 exp rounded to float32: 0.5
+// and 0.29; in float64 the exponentials took as long as the products around
+// them).  NaN in,
+// NaN out; below -104 the float32 result is 0.
+__device__ __forceinline__ float exp32(float x) {
+  const float c = x < -104.0f ? -104.0f : x;
+  const float n = __builtin_rintf(c * 1.44269504f);
+  float r = __builtin_fmaf(n, -0.693145752f, c);
+  r = __builtin_fmaf(n, -1.42860677e-06f, r);
+  float p = __builtin_fmaf(1.0f / 5040.0f, r, 1.0f / 720.0f);
+  p = __builtin_fmaf(p, r, 1.0f / 120.0f);
+  p = __builtin_fmaf(p, r, 1.0f / 24.0f);
+  p = __builtin_fmaf(p, r, 1.0f / 6.0f);
+  p = __builtin_fmaf(p, r, 0.5f);
+  return __builtin_ldexpf(1.0f + __builtin_fmaf(p, r * r, r), (int)n);
+}
+
+template <int HD>
+struct Fa {
+  static constexpr int HX = HD / 16;              // 16-wide column groups
+  static constexpr int P = HD + 4;                // LDS pitch: 16-byte aligned rows, conflict-free float4 reads
+  static constexpr int KS = HD <= 64 ? 64 : 32;   // rows per stage
+  static constexpr int RP = FA_NT / (HD / 4);     // rows per pass of the staging threads (a float4 each)
+  static constexpr int NL = (KS + RP - 1) / RP;   // passes
+};
+
+// four consecutive columns of a row at p, the first `n` of them valid
+__device__ __forceinline__ float4 fa_load4(const float *__restrict__ p, int n) {
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (n > 0) v.x = p[0];
+  if (n > 1) v.y = p[1];
+  if (n > 2) v.z = p[2];
+  if (n > 3) v.w = p[3];
+  return v;
+}
+
+// FULL (heads of exactly HD columns, 16-byte aligned): loads without guards,
+// rows past the end re-read the last one (their probabilities are 0 and their
+// results are not stored).  Otherwise columns past hd read as 0.
+
+// the lane's columns 16 x + 4*(l/16) .. +3 of row t
+template <int HD, bool FULL>
+__device__ __forceinline__ void fa_row(float4 (&v)[Fa<HD>::HX], const float *__restrict__ src, int t, int T, int D,
+                                       int hd, int lane) {
+  const int dl = 4 * (lane >> 4);
+  const float *p = src + (int64_t)min(t, T - 1) * D + dl;
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x)
+    v[x] = FULL ? *reinterpret_cast<const float4 *>(p + 16 * x) : fa_load4(p + 16 * x, hd - dl - 16 * x);
+}
+
+// Staging of rows [k0, k0 + KS) of one matrix: thread t brings column group
+// t % (HD / 4) of rows t / (HD / 4) + q RP.
+template <int HD, bool FULL>
+__device__ __forceinline__ void fa_fetch(float4 (&v)[Fa<HD>::NL], const float *__restrict__ src, int k0, int T, int D,
+                                         int hd) {
+  using F = Fa<HD>;
+  const int r = k0 + (int)threadIdx.x / (HD / 4), c = 4 * (threadIdx.x % (HD / 4));
+#pragma unroll
+  for (int q = 0; q < F::NL; ++q) {
+    const float *p = src + (int64_t)min(r + q * F::RP, T - 1) * D + c;
+    v[q] = FULL ? *reinterpret_cast<const float4 *>(p) : fa_load4(p, hd - c);
+  }
+}
+template <int HD>
+__device__ __forceinline__ void fa_put(float *dst, const float4 (&v)[Fa<HD>::NL]) {
+  using F = Fa<HD>;
+  const int r0 = threadIdx.x / (HD / 4), d = 4 * (threadIdx.x % (HD / 4));
+  if (FA_NT % (HD / 4) && r0 >= F::RP) return;
+#pragma unroll
+  for (int q = 0; q < F::NL; ++q)
+    if (F::KS % F::RP == 0 || r0 + q * F::RP < F::KS)
+      *reinterpret_cast<float4 *>(dst + (r0 + q * F::RP) * F::P + d) = v[q];
+}
+
+// acc[r] = sum_d Y[16 yt + 4*(l/16) + r][d] * Z[row][d], the lane's row in z
+template <int HD>
+__device__ __forceinline__ fx4 fa_tile(const float *sy, const float4 (&z)[Fa<HD>::HX], int yt, int lane) {
+  const float4 *p = reinterpret_cast<const float4 *>(sy + (16 * yt + (lane & 15)) * Fa<HD>::P + 4 * (lane >> 4));
+  // two chains, so a product does not wait for the one before it
+  fx4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x) {
+    const float4 y = p[4 * x];
+    a0 = mfma16(y.x, z[x].x, a0);
+    a1 = mfma16(y.y, z[x].y, a1);
+    a0 = mfma16(y.z, z[x].z, a0);
+    a1 = mfma16(y.w, z[x].w, a1);
+  }
+  return a0 + a1;
+}
+
+// o[x][r] += sum over the 16 rows j of tile yt of Y[j][16 x + 4*(l/16) + r] * zt[j] (the lane's column)
+template <int HD>
+__device__ __forceinline__ void fa_acc(fx4 (&o)[Fa<HD>::HX], const float *sy, const fx4 &zt, int yt, int lane) {
+  const float *p = sy + (16 * yt + 4 * (lane >> 4)) * Fa<HD>::P + (lane & 15);
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int x = 0; x < Fa<HD>::HX; ++x) o[x] = mfma16(p[s * Fa<HD>::P + 16 * x], zt[s], o[x]);
+}
+
+template <int HD, bool FULL>
+__device__ __forceinline__ void fa_store(float *__restrict__ G, const fx4 (&o)[Fa<HD>::HX], int64_t base, int t, int T,
+                                         int D, int hd, int lane) {
+  if (t >= T) return;
+  float *row = G + base + (int64_t)t * D;
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x) {
+    const int d = 16 * x + 4 * (lane >> 4);
+    if (FULL) {
+      *reinterpret_cast<float4 *>(row + d) = make_float4(o[x][0], o[x][1], o[x][2], o[x][3]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (d + r < hd) row[d + r] = o[x][r];
+    }
+  }
+}
+
+__device__ __forceinline__ float fa_max4(float v) {  // over the four lane groups
+  v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+__device__ __forceinline__ float fa_sum4(float v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
+// acc of the four waves added in wave order into wave 0's
+template <int HD>
+__device__ __forceinline__ void fa_merge(fx4 (&o)[Fa<HD>::HX], float *buf) {
+  constexpr int HX = Fa<HD>::HX;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float4 *b4 = reinterpret_cast<float4 *>(buf);
+  __syncthreads();
+  if (w > 0) {
+#pragma unroll
+    for (int x = 0; x < HX; ++x)
+      b4[((w - 1) * HX + x) * 64 + lane] = make_float4(o[x][0], o[x][1], o[x][2], o[x][3]);
+  }
+  __syncthreads();
+  if (w == 0) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int x = 0; x < HX; ++x) {
+        const float4 v = b4[(u * HX + x) * 64 + lane];
+        o[x] = o[x] + fx4{v.x, v.y, v.z, v.w};
+      }
+  }
+}
+
+// The diagonal of a 16 x 16 product tile: element (i, i) of lane column i.
+__device__ __forceinline__ float fa_diag(const fx4 &t, int lane) {
+  const int i = lane & 15;
+  const float v = (i & 3) == 0 ? t[0] : (i & 3) == 1 ? t[1] : (i & 3) == 2 ? t[2] : t[3];
+  return fa_sum4((lane >> 4) == (i >> 2) ? v : 0.f);
+}
+
+// d_i = gO_i . o_i through the instructions, and in the order, that form dP_ij
+// = gO_i . v_j: where a row has one key (o_i = v_j, P = 1) dP - d is then an
+// exact zero, as in the reference's sum over the row.
+template <int HD>
+__device__ __forceinline__ float fa_rowdot(const float4 (&o)[Fa<HD>::HX], const float4 (&g)[Fa<HD>::HX], int lane) {
+  fx4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x) {
+    a0 = mfma16(o[x].x, g[x].x, a0);
+    a1 = mfma16(o[x].y, g[x].y, a1);
+    a0 = mfma16(o[x].z, g[x].z, a0);
+    a1 = mfma16(o[x].w, g[x].w, a1);
+  }
+  return fa_diag(a0 + a1, lane);
+}
+
+// Block -> (pair, row block): the blocks of a pair are `npair` apart, so with
+// a multiple of 8 pairs they run on one XCD and share its L2; under the causal
+// mask the longest blocks are dispatched first.
+// SP: the four waves share 16 rows and take every fourth 16-row tile of the
+// other side (their results meet in LDS), which gives a short batch four times
+// the workgroups; otherwise each wave has 16 rows of its own.
+template <int HD, bool SP, bool FULL>
+__global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
+                                                       const float *__restrict__ V, float *__restrict__ O,
+                                                       float2 *__restrict__ st, int T, int D, int NH, int hd,
+                                                       int causal, int npair, int nb) {
+  using F = Fa<HD>;
+  constexpr int RB = SP ? 16 : FA_B;
+  __shared__ __align__(16) float sh[2 * F::KS * F::P];
+  __shared__ float wm[4][16], wl[4][16];
+  float *sk = sh, *sv = sh + F::KS * F::P;
+  const int pair = blockIdx.x % npair, qb = nb - 1 - blockIdx.x / npair;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t base = (int64_t)(pair / NH) * T * D + (pair % NH) * hd;
+  const int q0 = qb * RB + (SP ? 0 : 16 * w), qi = q0 + (lane & 15);
+  const float is = 1.0f / (float)sqrt((double)hd);
+  float4 qr[F::HX];
+  fa_row<HD, FULL>(qr, Q + base, qi, T, D, hd, lane);
+  fx4 o[F::HX];
+#pragma unroll
+  for (int x = 0; x < F::HX; ++x) o[x] = fx4{0.f, 0.f, 0.f, 0.f};
+  float m = -__builtin_inff(), l = 0.f;  // running maximum; the lane's own part of the sum
+  const int kend = causal ? min(T, qb * RB + RB) : T;
+  float4 kv[F::NL], vv[F::NL];
+  fa_fetch<HD, FULL>(kv, K + base, 0, T, D, hd);
+  fa_fetch<HD, FULL>(vv, V + base, 0, T, D, hd);
+  for (int k0 = 0; k0 < kend; k0 += F::KS) {
+    fa_put<HD>(sk, kv);
+    fa_put<HD>(sv, vv);
+    __syncthreads();
+    if (k0 + F::KS < kend) {
+      fa_fetch<HD, FULL>(kv, K + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, FULL>(vv, V + base, k0 + F::KS, T, D, hd);
+    }
+    const int jend = min(causal ? min(T, q0 + 16) : T, k0 + F::KS);  // the wave's live keys
+    auto mine = [&](int kt) { return k0 + 16 * kt < jend && (!SP || (((k0 >> 4) + kt) & 3) == w); };
+    bool any = false;
+#pragma unroll
+    for (int kt = 0; kt < F::KS / 16; ++kt) any = any || mine(kt);
+    if (any && q0 < T) {
+      fx4 s[F::KS / 16];
+      float mx = -__builtin_inff();
+#pragma unroll
+      for (int kt = 0; kt < F::KS / 16; ++kt) {
+        if (!mine(kt)) continue;
+        s[kt] = fa_tile<HD>(sk, qr, kt, lane);
+        const int jb = k0 + 16 * kt;
+        s[kt] = s[kt] * is;
+        if (jb + 15 >= T || (causal && jb + 15 > q0)) {  // uniform: a tile at an edge
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = jb + 4 * (lane >> 4) + r;
+            s[kt][r] = j >= T ? -__builtin_inff() : (causal && j > qi) ? -1e9f : s[kt][r];
+          }
+        }
+        mx = fmaxf(mx, fmaxf(fmaxf(s[kt][0], s[kt][1]), fmaxf(s[kt][2], s[kt][3])));
+      }
+      const float mn = fmaxf(m, fa_max4(mx));
+      const float ms = mn == -__builtin_inff() ? 0.f : mn;  // only -inf so far: weights 0
+      const float al = exp32(m - ms);
+      l *= al;
+#pragma unroll
+      for (int x = 0; x < F::HX; ++x) o[x] = o[x] * al;
+#pragma unroll
+      for (int kt = 0; kt < F::KS / 16; ++kt) {
+        if (!mine(kt)) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[kt][r] = exp32(s[kt][r] - ms);
+          l += s[kt][r];
+        }
+        fa_acc<HD>(o, sv, s[kt], kt, lane);
+      }
+      m = mn;
+    }
+    __syncthreads();
+  }
+  l = fa_sum4(l);
+  if (SP) {  // the waves' parts on a common maximum
+    if (lane < 16) wm[w][lane] = m;
+    __syncthreads();
+    const int i = lane & 15;
+    m = fmaxf(fmaxf(wm[0][i], wm[1][i]), fmaxf(wm[2][i], wm[3][i]));
+    const float f = exp32(wm[w][i] - (m == -__builtin_inff() ? 0.f : m));
+    if (lane < 16) wl[w][lane] = l * f;
+#pragma unroll
+    for (int x = 0; x < F::HX; ++x) o[x] = o[x] * f;
+    fa_merge<HD>(o, sh);
+    l = ((wl[0][i] + wl[1][i]) + wl[2][i]) + wl[3][i];
+    if (w > 0) return;
+  }
+  const float il = 1.0f / l;
+#pragma unroll
+  for (int x = 0; x < F::HX; ++x) o[x] = o[x] * il;
+  fa_store<HD, FULL>(O, o, base, qi, T, D, hd, lane);
+  if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = make_float2(m, il);
+}
+
+// Backward: gradScore = P (dP - d) / sqrt(hd), dP_ij = gO_i . v_j, d_i =
+// sum_j P_ij dP_ij = gO_i . o_i.  Two roles in one launch, each recomputing P
+// from the saved (maximum, 1 / sum), so every result has one writer and one
+// order of sums: key blocks (gK, gV over the live queries), dispatched first
+// as they do four products per tile pair, and query blocks (gQ over the live
+// keys, three products).
+template <int HD, bool SP, bool FULL>
+__global__ __launch_bounds__(FA_NT) void fa_bwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
+                                                       const float *__restrict__ V, const float *__restrict__ O,
+                                                       const float *__restrict__ GO, float *__restrict__ GQ,
+                                                       float *__restrict__ GK, float *__restrict__ GV,
+                                                       const float2 *__restrict__ st, int T, int D, int NH, int hd,
+                                                       int causal, int npair, int nb) {
+  using F = Fa<HD>;
+  constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
+  __shared__ __align__(16) float sh[2 * F::KS * F::P];
+  __shared__ __align__(16) float sm[F::KS], sl[F::KS], sd[F::KS];
+  float *sa = sh;                   // keys: K rows; queries: Q rows
+  float *sb = sh + F::KS * F::P;    // keys: V rows; queries: gO rows
+  const bool kside = (int)blockIdx.x < npair * nb;
+  const int bid = kside ? blockIdx.x : blockIdx.x - npair * nb;
+  const int pair = bid % npair, rb = kside ? bid / npair : nb - 1 - bid / npair;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, tid = threadIdx.x;
+  const int dl = 4 * (lane >> 4);
+  const int64_t base = (int64_t)(pair / NH) * T * D + (pair % NH) * hd;
+  const float is = 1.0f / (float)sqrt((double)hd);
+  const int r0 = rb * RB + (SP ? 0 : 16 * w), ri = r0 + (lane & 15);  // the wave's and the lane's row
+  const float2 *stp = st + (int64_t)pair * T;
+  float4 av[F::NL], bv[F::NL];
+  float4 za[F::HX], zb[F::HX], ov[F::HX];
+  fx4 ga[F::HX], gb[F::HX];
+#pragma unroll
+  for (int x = 0; x < F::HX; ++x) ga[x] = gb[x] = fx4{0.f, 0.f, 0.f, 0.f};
+  if (kside) {
+    fa_row<HD, FULL>(za, K + base, ri, T, D, hd, lane);
+    fa_row<HD, FULL>(zb, V + base, ri, T, D, hd, lane);
+    const int i0 = causal ? rb * RB / F::KS * F::KS : 0;  // first stage with a live query
+    // d and the saved statistics of a stage's queries: wave w its tile w
+    float2 ml;
+    auto fetch_rows = [&](int k0) {
+      if (w >= KT) return;
+      const int t = k0 + 16 * w + (lane & 15);
+      fa_row<HD, FULL>(ov, O + base, t, T, D, hd, lane);
+      ml = t < T ? stp[t] : make_float2(0.f, 0.f);  // rows past the end: probability 0
+    };
+    fa_fetch<HD, FULL>(av, Q + base, i0, T, D, hd);
+    fa_fetch<HD, FULL>(bv, GO + base, i0, T, D, hd);
+    fetch_rows(i0);
+    for (int k0 = i0; k0 < T; k0 += F::KS) {
+      fa_put<HD>(sa, av);
+      fa_put<HD>(sb, bv);
+      __syncthreads();
+      if (w < KT) {
+        float4 gr[F::HX];
+        const float4 *p = reinterpret_cast<const float4 *>(sb + (16 * w + (lane & 15)) * F::P + dl);
+#pragma unroll
+        for (int x = 0; x < F::HX; ++x) gr[x] = p[4 * x];
+        const float d = fa_rowdot<HD>(ov, gr, lane);
+        if (lane < 16) {
+          sm[16 * w + lane] = ml.x;
+          sl[16 * w + lane] = ml.y;
+          sd[16 * w + lane] = d;
+        }
+      }
+      if (k0 + F::KS < T) {
+        fa_fetch<HD, FULL>(av, Q + base, k0 + F::KS, T, D, hd);
+        fa_fetch<HD, FULL>(bv, GO + base, k0 + F::KS, T, D, hd);
+        fetch_rows(k0 + F::KS);
+      }
+      __syncthreads();
+      if (r0 < T) {
+#pragma unroll
+        for (int qt = 0; qt < KT; ++qt) {
+          const int ib = k0 + 16 * qt;
+          if (ib >= T || (causal && ib + 15 < r0) || (SP && ((ib >> 4) & 3) != w)) continue;  // uniform over the wave
+          fx4 s = fa_tile<HD>(sa, za, qt, lane), dp = fa_tile<HD>(sb, zb, qt, lane);
+          const float4 m4 = *reinterpret_cast<const float4 *>(sm + 16 * qt + dl);
+          const float4 l4 = *reinterpret_cast<const float4 *>(sl + 16 * qt + dl);
+          const float4 d4 = *reinterpret_cast<const float4 *>(sd + 16 * qt + dl);
+          const float mm[4] = {m4.x, m4.y, m4.z, m4.w}, ll[4] = {l4.x, l4.y, l4.z, l4.w};
+          const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+          fx4 ds;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[r] = exp32(s[r] * is - mm[r]) * ll[r];
+            ds[r] = s[r] * (dp[r] - dd[r]) * is;
+          }
+          if (ib + 15 >= T || r0 + 15 >= T || (causal && r0 + 15 > ib)) {  // uniform: a tile at an edge
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int i = ib + dl + r;
+              const bool live = i < T && ri < T && !(causal && ri > i);
+              s[r] = live ? s[r] : 0.f;
+              ds[r] = live ? ds[r] : 0.f;
+            }
+          }
+          fa_acc<HD>(gb, sb, s, qt, lane);   // gV_j += p_ij gO_i
+          fa_acc<HD>(ga, sa, ds, qt, lane);  // gK_j += gradScore_ij q_i
+        }
+      }
+      __syncthreads();
+    }
+    if (SP) {
+      fa_merge<HD>(ga, sh);
+      fa_merge<HD>(gb, sh);
+      if (w > 0) return;
+    }
+    fa_store<HD, FULL>(GK, ga, base, ri, T, D, hd, lane);
+    fa_store<HD, FULL>(GV, gb, base, ri, T, D, hd, lane);
+  } else {
+    fa_row<HD, FULL>(za, Q + base, ri, T, D, hd, lane);
+    fa_row<HD, FULL>(zb, GO + base, ri, T, D, hd, lane);
+    fa_row<HD, FULL>(ov, O + base, ri, T, D, hd, lane);
+    const float dsum = fa_rowdot<HD>(ov, zb, lane);
+    const float2 ml = ri < T ? stp[ri] : make_float2(0.f, 0.f);
+    const int kend = causal ? min(T, rb * RB + RB) : T;
+    fa_fetch<HD, FULL>(av, K + base, 0, T, D, hd);
+    fa_fetch<HD, FULL>(bv, V + base, 0, T, D, hd);
+    for (int k0 = 0; k0 < kend; k0 += F::KS) {
+      fa_put<HD>(sa, av);
+      fa_put<HD>(sb, bv);
+      __syncthreads();
+      if (k0 + F::KS < kend) {
+        fa_fetch<HD, FULL>(av, K + base, k0 + F::KS, T, D, hd);
+        fa_fetch<HD, FULL>(bv, V + base, k0 + F::KS, T, D, hd);
+      }
+      if (r0 < T) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const int jb = k0 + 16 * kt;
+          if (jb >= T || (causal && jb > r0 + 15) || (SP && ((jb >> 4) & 3) != w)) continue;
+          const fx4 s = fa_tile<HD>(sa, za, kt, lane), dp = fa_tile<HD>(sb, zb, kt, lane);
+          fx4 ds;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) ds[r] = exp32(s[r] * is - ml.x) * ml.y * (dp[r] - dsum) * is;
+          if (jb + 15 >= T || r0 + 15 >= T || (causal && jb + 15 > r0)) {  // uniform: a tile at an edge
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int j = jb + dl + r;
+              ds[r] = j < T && ri < T && !(causal && j > ri) ? ds[r] : 0.f;
+            }
+          }
+          fa_acc<HD>(ga, sa, ds, kt, lane);  // gQ_i += gradScore_ij k_j
+        }
+      }
+      __syncthreads();
+    }
+    if (SP) {
+      fa_merge<HD>(ga, sh);
+      if (w > 0) return;
+    }
+    fa_store<HD, FULL>(GQ, ga, base, ri, T, D, hd, lane);
+  }
+}
+
+static bool fa_supported(int D, int NH) { return NH > 0 && D % NH == 0 && D / NH <= 128; }
+
+size_t attn_work_floats(int B, int T, int D, int NH) {
+  return 2 * (size_t)B * NH * T * (fa_supported(D, NH) ? 1 : T);
+}
+
+template <int HD, bool SP, bool FULL>
+static hipError_t fa_launch(const float *Q, const float *K, const float *V, float *O, const float *GO, float *GQ,
+                            float *GK, float *GV, float *S, int B, int T, int D, int NH, int causal, hipStream_t s) {
+  const int hd = D / NH, rb = SP ? 16 : FA_B, nb = (T + rb - 1) / rb;
+  const int64_t np = (int64_t)B * NH;
+  if (np * nb * 2 > 0x7fffffff) return hipErrorInvalidValue;
+  float2 *st = reinterpret_cast<float2 *>(S);
+  if (!GO)
+    hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, FULL>), dim3((unsigned)(np * nb)), dim3(FA_NT), 0, s, Q, K, V, O, st, T,
+                       D, NH, hd, causal, (int)np, nb);
+  else
+    hipLaunchKernelGGL((fa_bwd_kernel<HD, SP, FULL>), dim3((unsigned)(2 * np * nb)), dim3(FA_NT), 0, s, Q, K, V, O, GO,
+                       GQ, GK, GV, st, T, D, NH, hd, causal, (int)np, nb);
+  return hipGetLastError();
+}
+
+// forward (GO null) or backward by head width, zero padded to the next of
+// 32, 48, 64, 80, 96 and 128
+static hipError_t fa_run(const float *Q, const float *K, const float *V, float *O, const float *GO, float *GQ,
+                         float *GK, float *GV, float *S, int B, int T, int D, int NH, int causal, hipStream_t s) {
+  const int hd = D / NH;
+  // up to 512 workgroups of 64 rows leave SIMDs with one wave or none: 16-row
+  // workgroups then (B 1, T 1024, one 64-wide head 229 -> 127 us; B 4, T 512,
+  // 8 heads 232 -> 216), not beyond (768 workgroups, B 2, T 1000, 12 heads:
+  // 293 -> 325), nor with 32-row stages, where half the waves would idle (80
+  // columns 160 -> 171), nor where the other side is a tile or two
+  const bool sp = T > 32 && (int64_t)B * NH * ((T + FA_B - 1) / FA_B) * (GO ? 2 : 1) <= 512;
+  uintptr_t al = reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+                 reinterpret_cast<uintptr_t>(O);
+  if (GO)
+    al |= reinterpret_cast<uintptr_t>(GO) | reinterpret_cast<uintptr_t>(GQ) | reinterpret_cast<uintptr_t>(GK) |
+          reinterpret_cast<uintptr_t>(GV);
+  const bool a16 = (al & 15) == 0;
+#define FA_CASE(H)                                                                                        \
+  if (hd <= H) {                                                                                          \
+    if (hd == H && a16)                                                                                   \
+      return sp && H <= 64                                                                                \
+                 ? fa_launch<H, (H <= 64), true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s)   \
+                 : fa_launch<H, false, true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);      \
+    return fa_launch<H, false, false>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);             \
+  }
+  FA_CASE(32);
+  FA_CASE(48);
+  FA_CASE(64);
+  FA_CASE(80);
+  FA_CASE(96);
+  FA_CASE(128);
+#undef FA_CASE
+  return hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------
+// Attention with heads wider than 128.  The scores of every (sample,
 // head) pair are materialised: S = Q_h K_h^T by one batched MFMA GEMM over
 // the B x NH pairs (each a T x hd slice of the [B*T, D] matrices), a row
 // kernel applies the mask, the scale and the reference's row softmax, and a
@@ -1608,7 +2120,6 @@ __global__ __launch_bounds__(256) void attn_dscore_rows(const float *__restrict_
   for (int j = lane; j < T; j += 64) g[j] = (causal && j > i) ? 0.f : (p[j] * (g[j] - d)) / scale;
 }
 
-size_t attn_gemm_floats(int B, int T, int NH) { return 2 * (size_t)B * NH * T * T; }
 
 namespace {
 // One batched GEMM over the (sample, head) pairs.  Operands are either a
@@ -1664,8 +2175,10 @@ hipError_t softmax_scores(float *S, int B, int T, int NH, int hd, int causal, hi
 }
 }  // namespace
 
-hipError_t launch_attn_fwd_gemm(const float *Q, const float *K, const float *V, float *O, int B, int T,
-                                int D, int NH, int causal, float *S, hipStream_t s) {
+hipError_t launch_attn_fwd_any(const float *Q, const float *K, const float *V, float *O, int B, int T,
+                               int D, int NH, int causal, float *S, hipStream_t s) {
+  if (fa_supported(D, NH))
+    return fa_run(Q, K, V, O, nullptr, nullptr, nullptr, nullptr, S, B, T, D, NH, causal, s);
   const int hd = D / NH;
   hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, S, true, B, T, D, NH, s);
   if (e == hipSuccess) e = softmax_scores(S, B, T, NH, hd, causal, s);
@@ -1673,9 +2186,11 @@ hipError_t launch_attn_fwd_gemm(const float *Q, const float *K, const float *V, 
   return e;
 }
 
-hipError_t launch_attn_bwd_gemm(const float *Q, const float *K, const float *V, const float *GO,
-                                float *GQ, float *GK, float *GV, int B, int T, int D, int NH, int causal,
-                                float *S, hipStream_t s) {
+hipError_t launch_attn_bwd_any(const float *Q, const float *K, const float *V, const float *O, const float *GO,
+                               float *GQ, float *GK, float *GV, int B, int T, int D, int NH, int causal,
+                               float *S, hipStream_t s) {
+  if (fa_supported(D, NH))
+    return fa_run(Q, K, V, const_cast<float *>(O), GO, GQ, GK, GV, S, B, T, D, NH, causal, s);
   const int hd = D / NH;
   float *P = S, *G = S + (size_t)B * NH * T * T;
   hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, P, true, B, T, D, NH, s);

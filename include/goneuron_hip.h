@@ -399,7 +399,8 @@ int gn_layernorm_backward(gn_ctx *ctx, const float *g, const float *x, const flo
  * wK | wV | wOut], each a Linear Dense (W D x D, b D).  work carries the
  * forward's saved state to the backward: gn_mha_workspace floats, the same
  * buffer and x for both calls.  Any T and head size: up to T = 128 and
- * 32-wide heads in fused kernels, beyond that through batched GEMMs over the
+ * 32-wide heads with a pair's rows in LDS, heads of up to 128 in kernels that
+ * stage the other side's rows, wider heads through batched GEMMs over the
  * materialised B x heads x T x T scores (included in the workspace); B x heads
  * must not exceed 65535. */
 int gn_mha_workspace(int32_t B, int32_t T, int32_t D, int32_t heads, int32_t use_rope,

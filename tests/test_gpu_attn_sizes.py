@@ -1,0 +1,77 @@
+"""Attention beyond the LDS-resident kernels (T > 128 or heads wider than 32), at
+the edges of its tiles and of its dispatch, against the oracle: head widths at
+and beside each padded width, sequences around the 16-row tiles, the 32/64-row
+stages and the 64-row workgroups, few (sample, head) pairs (16-row workgroups)
+and many.  Tolerance: the per-tensor 1e-4 of the reference's largest magnitude
+that every operator is held to."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from cfgutil import max_rel
+from gpuutil import DBuf, TOL, log
+
+pytestmark = pytest.mark.gpu
+
+
+def _mha(dev, B, T, D, NH, causal, p, x, g):
+    from goneuron_amd._lib import check, lib
+    L = lib()
+    ws = C.c_int64()
+    check(None, L.gn_mha_workspace(B, T, D, NH, 0, C.byref(ws)))
+    dx, dp, dg = DBuf(dev, x), DBuf(dev, p), DBuf(dev, g)
+    dout, dgr, dgin, dwk = (DBuf(dev, np.full(s, np.nan, np.float32))
+                            for s in ((B, T * D), p.shape, (B, T * D), ws.value))
+    check(dev.h, L.gn_mha_forward(dev.h, dx.p, dp.p, dout.p, dwk.p, B, T, D, NH, causal, 0))
+    check(dev.h, L.gn_mha_backward(dev.h, dx.p, dp.p, dg.p, dgr.p, dgin.p, dwk.p, B, T, D, NH, causal, 0,
+                                   C.c_float(np.float32(1) / np.float32(B))))
+    return dout.get(), dgr.get(), dgin.get()
+
+
+@pytest.mark.parametrize("B,T,D,NH,causal", [
+    (1, 129, 8, 2, 1), (2, 130, 15, 3, 0), (1, 191, 33, 1, 1), (2, 33, 48, 1, 0), (1, 65, 98, 2, 1),
+    (1, 64, 64, 1, 1), (2, 48, 63, 1, 0), (1, 193, 64, 1, 1), (1, 63, 80, 1, 0), (2, 31, 81, 1, 1),
+    (1, 97, 96, 1, 1), (1, 66, 128, 1, 0), (1, 17, 125, 1, 1), (1, 16, 130, 1, 0), (4, 1, 64, 1, 1),
+    (90, 65, 66, 2, 1), (140, 40, 128, 2, 0)])
+def test_attn_sizes(dev, oracle, B, T, D, NH, causal):
+    log(f"attention B={B} T={T} D={D} heads={NH} causal={causal}")
+    nd = min(B, 2)  # distinct samples; a larger batch repeats them
+    assert B % nd == 0
+    net = oracle.Net([oracle.spec(oracle.LAYER_MHA, dim=D, num_heads=NH, seq_len=T, causal=causal, use_rope=0)],
+                     oracle.LOSS_MSE)
+    rng = np.random.default_rng(T * D + NH)
+    p = (rng.normal(size=net.n) * (1.0 / np.sqrt(D))).astype(np.float32)
+    net.params[:] = p
+    x = rng.normal(size=(nd, T * D)).astype(np.float32)
+    g = rng.normal(size=(nd, T * D)).astype(np.float32)
+    out_r, gin_r = net.accumulate_grad(x, g, nd, T * D, T * D)
+    gr = net.grads.copy()
+    out, got, gin = _mha(dev, B, T, D, NH, causal, p, np.tile(x, (B // nd, 1)), np.tile(g, (B // nd, 1)))
+    for r in (0, B // nd - 1):
+        assert max_rel(out[r * nd:(r + 1) * nd], out_r) <= TOL
+        assert max_rel(gin[r * nd:(r + 1) * nd], gin_r) <= TOL
+    n1 = D * D + D
+    scale = np.abs(gr).max()
+    for i, name in enumerate(("wQ", "wK", "wV", "wOut")):
+        ref = gr[i * n1:(i + 1) * n1]
+        if np.abs(ref).max() <= 1e-6 * scale:  # sums that vanish (wK; wQ and wK at T = 1)
+            assert np.abs(got[i * n1:(i + 1) * n1]).max() <= 1e-5 * scale, name
+            continue
+        assert max_rel(got[i * n1:i * n1 + D * D], ref[:D * D]) <= TOL, name
+
+
+def test_attn_single_key_rows_have_no_score_gradient(dev):
+    """Under the causal mask token 0 attends to itself alone: its probability is
+    1 and gradScore an exact zero, so with a gradient on token 0 only the query
+    and key projections get exactly none (Adam would turn rounding noise there
+    into whole steps)."""
+    for T, D, NH in ((150, 64, 2), (40, 96, 1), (200, 128, 1), (70, 80, 2)):
+        rng = np.random.default_rng(T)
+        p = (rng.normal(size=4 * (D * D + D)) / np.sqrt(D)).astype(np.float32)
+        x = rng.normal(size=(3, T * D)).astype(np.float32)
+        g = np.zeros((3, T * D), np.float32)
+        g[:, :D] = rng.normal(size=(3, D))
+        _, got, _ = _mha(dev, 3, T, D, NH, 1, p, x, g)
+        assert not got[:2 * (D * D + D)].any(), (T, D, NH)
+        assert got[2 * (D * D + D):].any()
