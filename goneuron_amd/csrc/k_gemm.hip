@@ -28,12 +28,14 @@
 // epilogue.
 //
 // 128-wide tiles whose K ranges are whole stages run a four-wave variant
-// instead (gemm_f32_mfma_w4): one wave per 64 x 64 sub-tile over the whole K
-// range, operands fetched with direct global -> LDS loads (no staging
-// registers, no LDS store instructions), fragment reads and loads issued one
-// per MFMA.  With at least two tiles per CU it uses 32-deep stages so that two
-// blocks share a CU and one block's prologue, barriers and epilogue overlap
-// the other's MFMAs.
+// instead (gemm_f32_mfma_w4) where they belong to a forward pass: one wave per
+// 64 x 64 sub-tile over the whole K range, operands fetched with direct global
+// -> LDS loads (no staging registers, no LDS store instructions), fragment
+// reads and loads issued one per MFMA.  With at least two tiles per CU it uses
+// 32-deep stages so that two blocks share a CU and one block's prologue,
+// barriers and epilogue overlap the other's MFMAs.  Everywhere else those
+// tiles run on the bf16 matrix cores (gemm_split_bf16): each fp32 value as a
+// sum of three bf16, six partial products, an error below the fp32 MFMA's.
 //
 // Used by Dense forward (NT: X[B,in] * W[out,in]^T, fused bias + activation),
 // Dense dX (NN: dZ[B,out] * W[out,in], fused activation derivative of the layer
@@ -861,6 +863,255 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
   gemm_store<RM, RN, EPI, !AK, !BKC && TN == 2>(p, acc, m0, n0, wm, wn, half, l32);
 }
 
+// ---------------------------------------------------------------------------
+// The same product on the bf16 matrix cores, at better than fp32 accuracy: each
+// operand value is split into three bf16 parts, x = h + m + l exactly (8 + 8 +
+// 8 significant bits, round to nearest; below 2^-110 the last part underflows),
+// and a product is the six partial products down to 2^-16 of it (h h, h m, m h,
+// m m, h l, l h; what is left out is below 2^-26), by
+// v_mfma_f32_32x32x16_bf16.  These MFMAs run at 12 times the fp32 rate (1712
+// against 142 TFLOP/s measured from registers), so six of them per product
+// leave a ceiling of 285 TFLOP/s.
+//
+// They do not round their sum to nearest but down (a sum of K = 1024 positive
+// or negative products came out 2.2e-8 of its size too low, the fp32 MFMA's
+// 4e-10), which a later sum over many results would add up.  So only the 16 k
+// of a stage are summed there, from zero, smallest products first; the stage
+// sums are added in fp32 by the vector unit, and odd stages take -A and
+// subtract, which leaves the downward steps with alternating signs.  Against
+// float64 the error is 0.25 to 0.4 of the fp32 MFMA's (normal, positive, ReLU
+// and softmax-gradient operands, K 1024 and 4096), the mean error below 1e-10
+// but for the last (7e-9, of an error of 8e-8).
+//
+// Block tile 128 x 128, four waves of 64 x 64, K stages of 16 (one MFMA step,
+// 24 MFMAs per wave).  A stage's values go from global memory to registers
+// two stages before they are split there and written to LDS as three planes,
+// [row][16 k] in 16-byte chunks of 8 k (one lane's operand).  Four rows make a
+// 128-byte line whose 8 chunks swap by the line's parity, so both the writes
+// (2 chunks of 4 rows, or one chunk of 8) and the fragment reads (one chunk of
+// 8 rows) touch all banks.  Two LDS buffers (48 KB, so two blocks share a CU).
+// A stage's first half reads its second slabs of A and B, its second half the
+// first slabs of the next stage and writes the stage after that over this one,
+// one barrier between them.  Eight slices, each one MFMA at a time with a few
+// vector instructions or a read behind it: a wave issues in order, so what
+// stands behind two MFMAs waits for the first to leave the matrix pipe.  The
+// wave's 64 additions of stage sums beside ~100 vector instructions of
+// splitting keep the vector unit about as busy as the matrix pipe: 1024 x 4096
+// x 4096 NT takes 190 us (fp32 MFMAs 250), 182 with one running sum, 157 with
+// nothing but the MFMAs.
+//
+// Infinities and values whose rounding to bf16 overflows do not split
+// (inf - inf): a tile whose sums are not all finite is computed again on the
+// fp32 MFMA, which gives what the fp32 kernels give.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int SB_NT = 256;                 // threads
+constexpr int SB_BK = 16;                  // K per stage
+constexpr int SB_PL = 128 * SB_BK * 2;     // bytes of one plane of one operand
+constexpr int SB_OP = 3 * SB_PL;           // bytes of one operand's stage
+constexpr int SB_BUF = 2 * SB_OP;          // bytes of one stage
+
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+  const floatx2 v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+
+// values 2e, 2e + 1 of a chunk into its three planes
+__device__ __forceinline__ void split_pair(const float (&x)[8], int e, uintx4 (&o)[3], bool neg = false) {
+  const float a = neg ? -x[2 * e] : x[2 * e], b = neg ? -x[2 * e + 1] : x[2 * e + 1];
+  const unsigned h = bf16_pair(a, b);
+  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+  const unsigned m = bf16_pair(ra, rb);
+  const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
+  o[0][e] = h;
+  o[1][e] = m;
+  o[2][e] = bf16_pair(sa, sb);
+}
+
+// byte offset of chunk c (8 k) of a row inside a plane
+__device__ __forceinline__ int sb_off(int row, int c) {
+  const int line = row >> 2;
+  return line * 128 + (((((row & 3) << 1) | c) ^ (line & 1)) << 4);
+}
+
+// The thread's chunk of an operand's stage: K-contiguous, chunk tid & 1 of row
+// tid >> 1; otherwise chunk tid >> 7 of row tid & 127.
+template <bool KC>
+__device__ __forceinline__ int sb_row() {
+  return KC ? (int)threadIdx.x >> 1 : (int)threadIdx.x & 127;
+}
+template <bool KC>
+__device__ __forceinline__ int sb_chunk() {
+  return KC ? (int)threadIdx.x & 1 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 7);
+}
+// Its eight values of the stage at k0.  off: the start of the thread's row of a
+// K-contiguous operand, or its column otherwise (then the row addresses are
+// uniform over the wave and the loads need no alignment).
+template <bool KC>
+__device__ __forceinline__ void sb_load(const float *__restrict__ base, size_t off, int ld, int k0, float (&x)[8]) {
+  const int k = k0 + 8 * sb_chunk<KC>();
+  if (KC) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const floatx4 v = *reinterpret_cast<const floatx4 *>(base + off + k + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (base + (size_t)(k + e) * ld)[(unsigned)off];
+  }
+}
+
+// K a multiple of two stages; K-contiguous operands 16-byte
+// aligned with a pitch of a multiple of 4 (checked by the launcher).  K > 0.
+template <bool AK, bool BKC, int EPI>
+__global__ __launch_bounds__(SB_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_split_bf16(GemmArgs p, int tiles_m, int tiles_n) {
+  __shared__ __attribute__((aligned(16))) char sh[2 * SB_BUF];
+  batch_offsets(p);
+  int tm, tn;
+  tile_of_block(tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * 128, n0 = tn * 128;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 1, wn = w & 1;
+  const int nk = p.K / SB_BK;
+  floatx16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  // rows past the edge re-read the last one (their results are not stored)
+  const int ra = min(m0 + sb_row<AK>(), p.M - 1), rb = min(n0 + sb_row<BKC>(), p.N - 1);
+  const size_t ga = AK ? (size_t)ra * p.lda : (size_t)ra, gb = BKC ? (size_t)rb * p.ldb : (size_t)rb;
+  const int da = sb_off(sb_row<AK>(), sb_chunk<AK>()), db = SB_OP + sb_off(sb_row<BKC>(), sb_chunk<BKC>());
+  int fo[4];  // the lane's fragment offsets: two 32-row slabs of A, two of B
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    fo[i] = sb_off(64 * wm + 32 * i + (lane & 31), lane >> 5);
+    fo[2 + i] = SB_OP + sb_off(64 * wn + 32 * i + (lane & 31), lane >> 5);
+  }
+  float xa[2][8], xb[2][8];  // two stages of global loads in flight
+  auto load = [&](int t, int u) {  // past the last stage: that one again, never used
+    const int k0 = min(t, nk - 1) * SB_BK;
+    sb_load<AK>(p.A, ga, p.lda, k0, xa[u]);
+    sb_load<BKC>(p.B, gb, p.ldb, k0, xb[u]);
+  };
+  auto write = [&](char *S, const uintx4 (&o)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uintx4 *>(S + q * SB_PL) = o[q];
+  };
+  auto frag = [&](const char *S, int i, int q) { return *reinterpret_cast<const bf16x8 *>(S + q * SB_PL + fo[i]); };
+  load(0, 0);
+  load(1, 1);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    uintx4 oa[3], ob[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      split_pair(xa[u], e, oa, u);
+      split_pair(xb[u], e, ob);
+    }
+    write(sh + u * SB_BUF + da, oa);
+    write(sh + u * SB_BUF + db, ob);
+    load(2 + u, u);
+  }
+  __syncthreads();
+  bf16x8 f[5][3];  // [A 0, A 1, B 0, B 1, B 0 of odd stages][plane]
+#pragma unroll
+  for (int i = 0; i < 4; i += 2)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) f[i][q] = frag(sh, i, q);
+  for (int t = 0; t < nk; t += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};  // smallest products first
+      char *cur = sh + u * SB_BUF;               // stage t + u, then t + u + 2
+      const char *nxt = sh + (u ^ 1) * SB_BUF;  // stage t + u + 1
+      uintx4 oa[3], ob[3];
+      floatx16 s[2];  // the stage's sum of this tile and of the one before
+#pragma unroll
+      for (int sl = 0; sl < 8; ++sl) {
+        constexpr int TI[4] = {0, 0, 1, 1}, TJ[4] = {0, 1, 1, 0}, RD[8] = {3, 3, 1, 1, 0, 0, 2, 2};
+        const int ij = sl >> 1;
+        if (sl == 4) __syncthreads();
+        if (!(sl & 1))
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[ij & 1][r] = 0.f;
+#pragma unroll
+        for (int q = 3 * (sl & 1); q < 3 * (sl & 1) + 3; ++q)
+          s[ij & 1] =
+              __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[TI[ij]][PA[q]], f[TJ[ij] ? 3 : 2 + 2 * u][PB[q]], s[ij & 1], 0, 0, 0);
+#pragma unroll
+        for (int q = 2 * (sl & 1); q < 2 + (sl & 1); ++q) f[sl < 6 ? RD[sl] : 4 - 2 * u][q] = frag(sl < 4 ? cur : nxt, RD[sl], q);
+        if (sl < 4) split_pair(xa[u], sl, oa, u);
+        else split_pair(xb[u], sl - 4, ob);
+        if (sl == 4) write(cur + da, oa);
+        if (sl == 7) {
+          write(cur + db, ob);
+          load(t + u + 4, u);
+        }
+        if (sl >= 2) {  // half of the tile before
+          floatx16 &c = acc[TI[ij - 1]][TJ[ij - 1]];
+#pragma unroll
+          for (int r = 8 * (sl & 1); r < 8 * (sl & 1) + 8; ++r)
+            c[r] = u ? c[r] - s[(ij - 1) & 1][r] : c[r] + s[(ij - 1) & 1][r];
+        }
+        // masks: 0x008 MFMA, 0x002 vector, 0x100 LDS read, 0x200 LDS write
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[1][0][r] = u ? acc[1][0][r] - s[1][r] : acc[1][0][r] + s[1][r];
+    }
+  }
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad = bad || !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+  if (__syncthreads_or(bad)) {  // the whole tile again in fp32, operands straight from memory
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int k = lane >> 5; k < p.K; k += 2) {  // K is even
+      float a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = min(m0 + 64 * wm + 32 * i + (lane & 31), p.M - 1);
+        const int c = min(n0 + 64 * wn + 32 * i + (lane & 31), p.N - 1);
+        a[i] = p.A[AK ? (size_t)r * p.lda + k : (size_t)k * p.lda + r];
+        b[i] = p.B[BKC ? (size_t)c * p.ldb + k : (size_t)k * p.ldb + c];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  gemm_store<128, 128, EPI, false, false>(p, acc, m0, n0, wm, wn, lane >> 5, lane & 31);
+}
+
 // Split-K reduction: partials summed in split order, then the epilogue.
 // Blocks from nred on (p.cs_src set): the column sums cs_dst[c] = cs_scale *
 // sum_r cs_src[r][c], rows in order with eight loads in flight, one thread
@@ -932,22 +1183,40 @@ template <int R, bool AK, bool BKC, int EPI>
 static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int tn, int splits,
                           int kchunk, hipStream_t s) {
   dim3 grid(tm * tn, splits, a.nbatch > 1 ? a.nbatch : 1), block(NT);
-  if (R == 128 && vec && !ktail) {
+  // 128-wide tiles over whole 64-deep K stages.  Plain products and those of
+  // the backward pass (C = alpha A B, dX with its activation derivative): the
+  // split-bf16 kernel (1024 x 4096 x 4096 NN 251 -> 202 us, 4096 x 4096 x 1024
+  // TN 261 -> 201, error 1.14e-6 -> 2.9e-7 and 5.7e-7 -> 1.5e-7).  A forward
+  // pass (bias, activation) keeps its order of fp32 sums: any other changes
+  // which units within rounding of 0 pass their ReLU, which moves a layer's
+  // gradient by 1e-3, where the split in the backward pass moves it by 1e-6.
+  // 64-wide tiles stay with eight waves of fp32 MFMAs, mostly faster there
+  // (4096 x 256 x 1024 22 against 28 us).
+  if constexpr (R == 128 && (EPI == EPI_SCALE || EPI == EPI_DACT)) {
+    if (vec && !ktail) {
+      hipLaunchKernelGGL((gemm_split_bf16<AK, BKC, EPI>), grid, dim3(SB_NT), 0, s, a, tm, tn);
+      return hipGetLastError();
+    }
+  } else if constexpr (R == 128) {
     // Four-wave kernels: 32-deep stages (64 KB of LDS) when there are at
     // least two tiles per CU (two blocks share a CU) or the K range is at most
     // four 64-deep stages (the transformer's K = 256 projections: +0.7 % on
     // its step; at K = 1024 the C3 step lost 3 %); else 64-deep stages, one
     // block per CU.
-    if (tm * tn * splits >= 512 || kchunk <= 256)
-      hipLaunchKernelGGL((gemm_f32_mfma_w4<32, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn,
-                         kchunk);
-    else
-      hipLaunchKernelGGL((gemm_f32_mfma_w4<64, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn,
-                         kchunk);
-  } else if (vec && !ktail)
-    hipLaunchKernelGGL((gemm_f32_mfma<R, AK, BKC, true, EPI, 1>), grid, block, 0, s, a, tm, tn,
-                       kchunk);
-  else if (vec)
+    if (vec && !ktail) {
+      if (tm * tn >= 512 || kchunk <= 256)
+        hipLaunchKernelGGL((gemm_f32_mfma_w4<32, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn, kchunk);
+      else
+        hipLaunchKernelGGL((gemm_f32_mfma_w4<64, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn, kchunk);
+      return hipGetLastError();
+    }
+  } else {
+    if (vec && !ktail) {
+      hipLaunchKernelGGL((gemm_f32_mfma<R, AK, BKC, true, EPI, 1>), grid, block, 0, s, a, tm, tn, kchunk);
+      return hipGetLastError();
+    }
+  }
+  if (vec)
     hipLaunchKernelGGL((gemm_f32_mfma<R, AK, BKC, true, EPI, 2>), grid, block, 0, s, a, tm, tn,
                        kchunk);
   else
@@ -975,7 +1244,8 @@ static hipError_t launch_r(char ta, char tb, int epi, bool vec, const GemmArgs &
   // float4-legal operands take the pipelined loop; it checks k only when the
   // last K stage is partial
   const bool ktail = a.K % BK != 0;
-  if (splits > 1) return launch_e<R, EPI_PARTIAL>(ta, tb, vec, ktail, a, tm, tn, splits, kchunk, s);
+  if constexpr (R == 64)  // a grid that takes 128-wide tiles fills the chip without a split
+    if (splits > 1) return launch_e<R, EPI_PARTIAL>(ta, tb, vec, ktail, a, tm, tn, splits, kchunk, s);
   if (epi == EPI_BIAS_ACT)
     return launch_e<R, EPI_BIAS_ACT>(ta, tb, vec, ktail, a, tm, tn, 1, kchunk, s);
   if (epi == EPI_DACT) return launch_e<R, EPI_DACT>(ta, tb, vec, ktail, a, tm, tn, 1, kchunk, s);
@@ -1031,7 +1301,7 @@ hipError_t launch_gemm(char ta, char tb, int epi, const GemmArgs &a0, hipStream_
   // short K (at most four 64-deep stages) with four 64-wide tiles per CU:
   // 64-wide tiles, whose blocks cover each other's prologue and epilogue
   const bool big = plan_big(a);
-  if (a.kseg > 0 && big) return hipErrorNotSupported;  // the four-wave kernels load whole K ranges
+  if (a.kseg > 0 && big) return hipErrorNotSupported;  // the 128-wide kernels load whole K ranges
   const int tiles = (int)std::min<int64_t>(big ? t128 : t64, 1 << 30);
   int splits = 1;
   if (tiles < 160 && a.K >= 8 * BK && a.ws) {
