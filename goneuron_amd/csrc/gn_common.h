@@ -550,16 +550,18 @@ hipError_t launch_ln_bwd_part(const float *g, const float *gpool, int poolT, con
                               const float *gam, const float *stats, float *dx, float *part, float *tsum,
                               int rows, int N, hipStream_t s, const float *tsx = nullptr,
                               float *tss = nullptr, int tsB = 0, int tsT = 0, int tsN = 0);
-hipError_t launch_ln_bwd(const float *g, const float *x, const float *gam, const float *stats,
-                         float *dx, float *gx, int rows, int N, hipStream_t s);
+hipError_t launch_ln_bwd(const float *g, const float *x, const float *gam, const float *stats, float *dx,
+                         float *dgam, float *dbet, float *work, int rows, int N, float scale, float *ws,
+                         size_t ws_cap, hipStream_t s);
 // Rotary embedding of rows [rows, NH*hd] in place; position = row % T; cs/sn
 // are [T][hd/2] tables; conj rotates the other way.
 hipError_t launch_rope(float *x, const float *cs, const float *sn, int rows, int T, int NH, int hd,
                        int conj, hipStream_t s);
 hipError_t launch_rms_fwd(const float *x, const float *gam, float *y, float *rms, int rows, int N,
                           float eps, hipStream_t s);
-hipError_t launch_rms_bwd(const float *g, const float *x, const float *gam, const float *rms,
-                          float *dx, float *gx, int rows, int N, hipStream_t s);
+hipError_t launch_rms_bwd(const float *g, const float *x, const float *gam, const float *rms, float *dx,
+                          float *dgam, float *work, int rows, int N, float scale, float *ws, size_t ws_cap,
+                          hipStream_t s);
 bool attn_supported(int T, int D, int NH);  // the fused kernels: T <= 128, D / NH <= 32
 // Attention of any T and head size: heads of up to 128 in kernels that stage
 // the other side's rows, wider ones through batched GEMMs over the (sample,

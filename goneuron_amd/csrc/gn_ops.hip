@@ -205,8 +205,8 @@ extern "C" int gn_softmax_ce_backward(gn_ctx *c, float *zo, const float *y, floa
 // LayerNorm (layernorm.go:193-441) over rows of N: y = gamma (x - mean) / std
 // + beta with std = sqrt(var + eps) (eps 0 selects 1e-5); stats keeps (mean,
 // std) per row for the backward, whose dx follows the reference's formula
-// (its last term uses N std^2; Q18).  work: rows x N floats of scratch for
-// g * xhat.  dgamma / dbeta = scale * sums over the rows.
+// (its last term uses N std^2; Q18).  work: rows x N floats of scratch, for
+// g * xhat of rows of more than 2048.  dgamma / dbeta = scale * sums over the rows.
 // ---------------------------------------------------------------------------
 extern "C" int gn_layernorm_forward(gn_ctx *c, const float *x, const float *gamma, const float *beta,
                                     float *y, float *stats, int32_t rows, int32_t N, float eps) {
@@ -224,14 +224,9 @@ extern "C" int gn_layernorm_backward(gn_ctx *c, const float *g, const float *x, 
   ENTRY(c);
   if (!g || !x || !gamma || !stats || !dx || !dgamma || !dbeta || !work || rows <= 0 || N <= 0)
     return set_err(c, GN_ERR_INVALID, "bad layernorm args");
-  {
-    KTimer kt(c, GN_KCLASS_OTHER, "ln_bwd", f4(4.0 * rows * N + 2.0 * rows));
-    HIP_OK(c, launch_ln_bwd(g, x, gamma, stats, dx, work, rows, N, c->stream));
-  }
-  const float *src[2] = {work, g};
-  float *dst[2] = {dgamma, dbeta};
-  KTimer kt(c, GN_KCLASS_OTHER, "colsum", 2 * f4((double)rows * N + N));
-  HIP_OK(c, launch_colsum_multi(src, dst, 2, rows, N, N, scale, c->scratch, c->scratch_floats, c->stream));
+  KTimer kt(c, GN_KCLASS_OTHER, "ln_bwd", f4(3.0 * rows * N + 2.0 * rows + 2.0 * N));
+  HIP_OK(c, launch_ln_bwd(g, x, gamma, stats, dx, dgamma, dbeta, work, rows, N, scale, c->scratch,
+                          c->scratch_floats, c->stream));
   return GN_OK;
 }
 
@@ -664,7 +659,7 @@ extern "C" int gn_avgpool2d_backward(gn_ctx *c, const float *gout, float *gin, i
 // RMSNorm (rmsnorm.go:222-329) over rows of N: y = gamma x / rms, rms =
 // sqrt(mean(x^2) + eps) (eps 0 selects 1e-5); the backward is the
 // reference's formula (its projection term is scaled by gamma_j, Q19).
-// work: rows x N floats (g x / rms for the gamma sums).
+// work: rows x N floats (g x / rms for the gamma sums of rows of more than 2048).
 // ---------------------------------------------------------------------------
 extern "C" int gn_rmsnorm_forward(gn_ctx *c, const float *x, const float *gamma, float *y, float *rms,
                                   int32_t rows, int32_t N, float eps) {
@@ -682,12 +677,9 @@ extern "C" int gn_rmsnorm_backward(gn_ctx *c, const float *g, const float *x, co
   ENTRY(c);
   if (!g || !x || !gamma || !rms || !dgamma || !work || rows <= 0 || N <= 0)
     return set_err(c, GN_ERR_INVALID, "bad rmsnorm args");
-  {
-    KTimer kt(c, GN_KCLASS_OTHER, "rms_bwd", f4(4.0 * rows * N + rows));
-    HIP_OK(c, launch_rms_bwd(g, x, gamma, rms, dx, work, rows, N, c->stream));
-  }
-  KTimer kt(c, GN_KCLASS_OTHER, "colsum", f4((double)rows * N + N));
-  HIP_OK(c, launch_colsum(work, rows, N, N, scale, dgamma, c->scratch, c->scratch_floats, c->stream));
+  KTimer kt(c, GN_KCLASS_OTHER, "rms_bwd", f4(3.0 * rows * N + rows + N));
+  HIP_OK(c, launch_rms_bwd(g, x, gamma, rms, dx, dgamma, work, rows, N, scale, c->scratch, c->scratch_floats,
+                           c->stream));
   return GN_OK;
 }
 

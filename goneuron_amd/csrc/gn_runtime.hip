@@ -1654,22 +1654,12 @@ static hipError_t tb_norm_bwd(gn_ctx *c, const LayerRT &R, const float *P, float
     if (e != hipErrorNotSupported) return e;
     (void)hipGetLastError();
   }
-  {
-    // read g, x and the statistics, write dx and g * xhat
-    KTimer kt(c, GN_KCLASS_OTHER, rms ? "rms_bwd" : "ln_bwd", f4(4.0 * rows * D + (rms ? 1 : 2) * rows));
-    if (rms) {
-      e = launch_rms_bwd(g, x, P + og, st, dx, t.GX, rows, D, c->stream);
-    } else {
-      e = launch_ln_bwd(g, x, P + og, st, dx, t.GX, rows, D, c->stream);
-    }
-  }
-  if (e != hipSuccess) return e;
-  // gamma (and for LayerNorm beta) gradients in one launch pair
-  const float *src[2] = {t.GX, g};
-  float *dst[2] = {G + og, G + ob};
-  const int nm = rms ? 1 : 2;
-  KTimer kt(c, GN_KCLASS_OTHER, "colsum", nm * f4((double)rows * D + D));
-  return launch_colsum_multi(src, dst, nm, rows, D, D, scale, c->scratch, c->scratch_floats, c->stream);
+  KTimer kt(c, GN_KCLASS_OTHER, rms ? "rms_bwd" : "ln_bwd", f4(3.0 * rows * D + (rms ? 1 : 2) * (rows + D)));
+  if (rms)
+    return launch_rms_bwd(g, x, P + og, st, dx, G + og, t.GX, rows, D, scale, c->scratch, c->scratch_floats,
+                          c->stream);
+  return launch_ln_bwd(g, x, P + og, st, dx, G + og, G + ob, t.GX, rows, D, scale, c->scratch, c->scratch_floats,
+                       c->stream);
 }
 
 // cls (may be null): the output of a CLSPooling above, written by norm 2
@@ -2494,17 +2484,11 @@ static int model_backward(gn_model *M, const float *x, int B, float scale, const
           e = launch_ln_bwd_params(R.gout, in, gam, R.rmsv, dx, dg, db, rows, N, scale, c->scratch,
                                    c->scratch_floats, c->stream);
         }
-        if (e == hipErrorNotSupported) {  // partials beyond the scratch: g * xhat, then column sums
+        if (e == hipErrorNotSupported) {  // more than 512 columns, or partials beyond the scratch
           (void)hipGetLastError();
-          {
-            KTimer kt(c, GN_KCLASS_OTHER, "ln_bwd", f4(4.0 * rows * N + 2.0 * rows));
-            HIP_OK(c, launch_ln_bwd(R.gout, in, gam, R.rmsv, dx, R.gx, rows, N, c->stream));
-          }
-          const float *src[2] = {R.gx, R.gout};
-          float *dst[2] = {dg, db};
-          KTimer kt(c, GN_KCLASS_OTHER, "colsum", 2 * f4((double)rows * N + N));
-          HIP_OK(c, launch_colsum_multi(src, dst, 2, rows, N, N, scale, c->scratch, c->scratch_floats,
-                                        c->stream));
+          KTimer kt(c, GN_KCLASS_OTHER, "ln_bwd", f4(3.0 * rows * N + 2.0 * rows + 2.0 * N));
+          HIP_OK(c, launch_ln_bwd(R.gout, in, gam, R.rmsv, dx, dg, db, R.gx, rows, N, scale, c->scratch,
+                                  c->scratch_floats, c->stream));
         } else {
           HIP_OK(c, e);
         }
@@ -2645,12 +2629,11 @@ static int model_backward(gn_model *M, const float *x, int B, float scale, const
         break;
       }
       case GN_LAYER_RMSNORM: {  // rmsnorm.go:301-329: dx, then gamma += g * (x / rms)
-        KTimer kt(c, GN_KCLASS_OTHER, "rms_bwd", f4(5.0 * B * R.in_len));
         const int rows = B * (R.in_len / R.D);
+        KTimer kt(c, GN_KCLASS_OTHER, "rms_bwd", f4(3.0 * B * R.in_len + rows + R.D));
         HIP_OK(c, launch_rms_bwd(R.gout, in, M->params + R.poff, R.rmsv, below ? below->gout : nullptr,
-                                 R.gx, rows, R.D, c->stream));
-        HIP_OK(c, launch_colsum(R.gx, rows, R.D, R.D, scale, M->grads + R.poff, c->scratch,
-                                c->scratch_floats, c->stream));
+                                 M->grads + R.poff, R.gx, rows, R.D, scale, c->scratch, c->scratch_floats,
+                                 c->stream));
         is_dz = false;
         break;
       }

@@ -391,7 +391,7 @@ int gn_layernorm_forward(gn_ctx *ctx, const float *x, const float *gamma, const 
                          float *y, float *stats, int32_t rows, int32_t N, float eps);
 /* LayerNorm.Backward (layernorm.go:334-441): dx by the reference's formula
  * (its last term divides by N std^2), dgamma = scale * sum g * xhat, dbeta =
- * scale * sum g; work = rows x N floats of scratch. */
+ * scale * sum g; work = rows x N floats of scratch (used where N > 2048). */
 int gn_layernorm_backward(gn_ctx *ctx, const float *g, const float *x, const float *gamma,
                           const float *stats, float *dx, float *dgamma, float *dbeta, float *work,
                           int32_t rows, int32_t N, float scale);
@@ -463,7 +463,7 @@ int gn_avgpool2d_backward(gn_ctx *ctx, const float *gout, float *gin, int32_t B,
 /* RMSNorm.ForwardWithArena / Backward (rmsnorm.go:222-329) over `rows` rows of
  * N: y = gamma x / rms, rms per row for the backward (eps 0 selects 1e-5);
  * dx (may be NULL) follows the reference's formula; dgamma = scale * sums;
- * work: rows x N floats. */
+ * work: rows x N floats of scratch (used where N > 2048). */
 int gn_rmsnorm_forward(gn_ctx *ctx, const float *x, const float *gamma, float *y, float *rms,
                        int32_t rows, int32_t N, float eps);
 int gn_rmsnorm_backward(gn_ctx *ctx, const float *g, const float *x, const float *gamma, const float *rms,
