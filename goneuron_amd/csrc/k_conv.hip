@@ -630,6 +630,95 @@ __global__ __launch_bounds__(CT) void conv3_fwd_group_kernel(const float *__rest
   }
 }
 
+// Forward with K x K taps and any number of input channels: a thread per output
+// position and OCG output channels.  conv2d_fwd_kernel, a channel per thread,
+// reads every tap once per output channel and is bound by those loads; here a
+// position's window of one input channel is read once into registers (rows and
+// columns outside the plane from clamped addresses) and serves OCG channels,
+// whose weights are uniform and come through scalar loads, so what is left is
+// the multiplies and adds.  Each output keeps conv2d_fwd_kernel's expressions in
+// its order: the same bits.  FAST: k3 s1 p1.
+template <int K, int OCG, bool FAST>
+__global__ __launch_bounds__(CT) void conv_fwd_oc_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                         const float *__restrict__ bias, float *__restrict__ out,
+                                                         ConvShape s, int fwd) {
+  const int osz = s.oH * s.oW, pos = blockIdx.x * CT + threadIdx.x;
+  if (pos >= osz) return;
+  const int groups = (s.outC + OCG - 1) / OCG;
+  const int o0 = (int)(blockIdx.y % groups) * OCG, b = blockIdx.y / groups;
+  const int oh = pos / s.oW, ow = pos - oh * s.oW, plane = s.H * s.W;
+  int ro[K], co[K];
+  bool rok[K], cok[K];
+#pragma unroll
+  for (int t = 0; t < K; ++t) {
+    const int ih = oh * s.stride + t - s.pad, iw = ow * s.stride + t - s.pad;
+    rok[t] = ih >= 0 && ih < s.H;
+    cok[t] = iw >= 0 && iw < s.W;
+    ro[t] = min(max(ih, 0), s.H - 1) * s.W;
+    co[t] = min(max(iw, 0), s.W - 1);
+  }
+  const bool inner = FAST && oh >= 1 && oh < s.oH - 1;
+  const float *xs = x + (int64_t)b * s.inC * plane;
+  float p[OCG];
+#pragma unroll
+  for (int j = 0; j < OCG; ++j) p[j] = 0.f;
+  for (int ic = 0; ic < s.inC; ++ic, xs += plane) {
+    float v[K][K];
+#pragma unroll
+    for (int r = 0; r < K; ++r)
+#pragma unroll
+      for (int c = 0; c < K; ++c) v[r][c] = xs[ro[r] + co[c]];
+    if (inner) {
+      if constexpr (FAST) {
+#pragma unroll
+        for (int j = 0; j < OCG; ++j) {
+          const float *wk = w + ((int64_t)min(o0 + j, s.outC - 1) * s.inC + ic) * 9;
+#pragma unroll
+          for (int r = 0; r < 3; ++r) p[j] += wk[3 * r] * v[r][0] + wk[3 * r + 1] * v[r][1] + wk[3 * r + 2] * v[r][2];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < OCG; ++j) {
+        const float *wk = w + ((int64_t)min(o0 + j, s.outC - 1) * s.inC + ic) * (K * K);
+#pragma unroll
+        for (int r = 0; r < K; ++r)
+#pragma unroll
+          for (int c = 0; c < K; ++c) {
+            const float t = p[j] + wk[r * K + c] * v[r][c];
+            p[j] = rok[r] && cok[c] ? t : p[j];
+          }
+      }
+    }
+  }
+  // Q7: the edge columns of interior rows keep 0
+  const bool drop = inner && (ow < 1 || ow >= s.oW - 1);
+#pragma unroll
+  for (int j = 0; j < OCG; ++j) {
+    const int oc = o0 + j;
+    if (oc >= s.outC) break;
+    const float z = (drop ? 0.f : p[j]) + bias[oc];
+    out[((int64_t)b * s.outC + oc) * osz + pos] =
+        fwd == F_RELU ? (z > 0.0f ? z : 0.0f) : fwd == F_IDENTITY ? z : act_fwd_call(z, fwd);
+  }
+}
+
+template <int K, bool FAST>
+static hipError_t conv_fwd_oc(const float *x, const float *w, const float *bias, float *out, const ConvShape &s, int B,
+                              int fwd, hipStream_t st) {
+  // eight channels per thread where that still leaves four waves per SIMD
+  // (1024 workgroups), else four
+  const unsigned gx = (unsigned)((s.oH * s.oW + CT - 1) / CT);
+  const int64_t g8 = (s.outC + 7) / 8;
+  if ((int64_t)gx * B * g8 >= 1024)
+    hipLaunchKernelGGL((conv_fwd_oc_kernel<K, 8, FAST>), dim3(gx, (unsigned)(B * g8)), dim3(CT), 0, st, x, w, bias, out,
+                       s, fwd);
+  else
+    hipLaunchKernelGGL((conv_fwd_oc_kernel<K, 4, FAST>), dim3(gx, (unsigned)(B * ((s.outC + 3) / 4))), dim3(CT), 0, st,
+                       x, w, bias, out, s, fwd);
+  return hipGetLastError();
+}
+
 template <int INC>
 static hipError_t conv3_fwd_inc(const float *x, const float *w, const float *bias, float *out,
                                 const ConvShape &s, int B, int fwd, float *pout, int32_t *parg,
@@ -681,6 +770,12 @@ hipError_t launch_conv_fwd(const float *x, const float *w, const float *bias, fl
     }
   }
   if (pool_out) return hipErrorInvalidValue;
+  if (s.H >= 1 && s.W >= 1 && s.oH >= 1 && s.oW >= 1 && (int64_t)B * s.outC <= 65535 && s.outC >= 4) {
+    if (s.k == 3 && s.stride == 1 && s.pad == 1) return conv_fwd_oc<3, true>(x, w, bias, out, s, B, fwd, st);
+    if (s.k == 3) return conv_fwd_oc<3, false>(x, w, bias, out, s, B, fwd, st);
+    if (s.k == 1) return conv_fwd_oc<1, false>(x, w, bias, out, s, B, fwd, st);
+    if (s.k == 5) return conv_fwd_oc<5, false>(x, w, bias, out, s, B, fwd, st);
+  }
   const int osz = s.oH * s.oW;
   const int gx = std::min((osz + CT - 1) / CT, 64);
   hipLaunchKernelGGL(conv2d_fwd_kernel, dim3(gx, B * s.outC), dim3(CT), 0, st, x, w, bias, out, s, B,
