@@ -373,6 +373,35 @@ __global__ __launch_bounds__(CT) void conv2d_wgrad_mfma(const float *__restrict_
     }
 }
 
+// Many slots: a workgroup sums 32 of them, each half wave every 32nd block's row
+// (whole 128-byte lines, eight in flight; a wave per slot reads one value of each
+// line: 1024 blocks of 4640 slots 27 us of a 120 us layer, now 99 in all), and
+// the 32 sums of a slot are added in a fixed order.
+constexpr int WR_S = 32, WR_NT = 1024, WR_H = WR_NT / WR_S;
+__global__ __launch_bounds__(WR_NT) void conv2d_wgrad_reduce_rows(const float *__restrict__ part, int nblocks,
+                                                                  int nslots, float scale, float *__restrict__ grad) {
+  __shared__ float red[WR_H][WR_S + 1];
+  const int c = threadIdx.x & (WR_S - 1), h = threadIdx.x / WR_S, o = blockIdx.x * WR_S + c;
+  float s = 0.f;
+  if (o < nslots)
+    for (int i = h; i < nblocks; i += 8 * WR_H) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = i + WR_H * u < nblocks ? part[(int64_t)(i + WR_H * u) * nslots + o] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (i + WR_H * u < nblocks) s += v[u];
+    }
+  red[h][c] = s;
+  __syncthreads();
+  // half wave h now holds slot h's sums, one per lane
+  s = red[c][h];
+#pragma unroll
+  for (int d = WR_H / 2; d > 0; d >>= 1) s += __shfl_xor(s, d, WR_H);
+  const int slot = blockIdx.x * WR_S + h;
+  if (c == 0 && slot < nslots) grad[slot] = s * scale;  // [dW | db]
+}
+
 // One wave per slot: lanes take the blocks, then a wave reduction.  With the
 // step's update (ad.stride), each slot's gradient is updated by the lane that
 // writes it, and blocks from nred on update ad.rest's ranges.
@@ -893,6 +922,18 @@ hipError_t launch_conv_wgrad_reduce(const ConvWgradReduce &red, const AdamStep *
   return hipGetLastError();
 }
 
+// From 2048 slots on (64 workgroups) by rows; below, a wave per slot keeps more
+// loads in flight (448 slots in 14 workgroups of rows: the CNN step 58.6 -> 63 us).
+static hipError_t conv_wgrad_sum(const float *ws, int nblocks, int nslots, float scale, float *grad, hipStream_t st) {
+  if (nslots >= 2048)
+    hipLaunchKernelGGL(conv2d_wgrad_reduce_rows, dim3((nslots + WR_S - 1) / WR_S), dim3(WR_NT), 0, st, ws, nblocks,
+                       nslots, scale, grad);
+  else
+    hipLaunchKernelGGL(conv2d_wgrad_reduce, dim3((nslots + 3) / 4), dim3(CT), 0, st, ws, nblocks, nslots, scale, grad,
+                       (nslots + 3) / 4, AdamStep{});
+  return hipGetLastError();
+}
+
 hipError_t launch_conv_wgrad(const float *x, const float *gout, const float *out, float *grad,
                              const ConvShape &s, int B, int deriv, float scale, float *ws,
                              size_t ws_cap, hipStream_t st, ConvWgradReduce *red) {
@@ -916,9 +957,7 @@ hipError_t launch_conv_wgrad(const float *x, const float *gout, const float *out
       *red = ConvWgradReduce{ws, nblocks, nslots, scale, grad};
       return hipGetLastError();
     }
-    hipLaunchKernelGGL(conv2d_wgrad_reduce, dim3((nslots + 3) / 4), dim3(CT), 0, st, ws, nblocks,
-                       nslots, scale, grad, (nslots + 3) / 4, AdamStep{});
-    return hipGetLastError();
+    return conv_wgrad_sum(ws, nblocks, nslots, scale, grad, st);
   }
   // scalar path for shapes whose input rows do not fit: dz tile <= 32 KiB
   band = s.oH;
@@ -933,9 +972,7 @@ hipError_t launch_conv_wgrad(const float *x, const float *gout, const float *out
     *red = ConvWgradReduce{ws, nblocks, nslots, scale, grad};
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(conv2d_wgrad_reduce, dim3((nslots + 3) / 4), dim3(CT), 0, st, ws, nblocks,
-                     nslots, scale, grad, (nslots + 3) / 4, AdamStep{});
-  return hipGetLastError();
+  return conv_wgrad_sum(ws, nblocks, nslots, scale, grad, st);
 }
 
 hipError_t launch_conv_dgrad(const float *gout, const float *out, const float *w, float *gin,
