@@ -866,10 +866,13 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
 // ---------------------------------------------------------------------------
 // The same product on the bf16 matrix cores, at better than fp32 accuracy: each
 // operand value is split into three bf16 parts, x = h + m + l exactly (8 + 8 +
-// 8 significant bits, round to nearest; below 2^-110 the last part underflows),
-// and a product is the six partial products down to 2^-16 of it (h h, h m, m h,
-// m m, h l, l h; what is left out is below 2^-26), by
-// v_mfma_f32_32x32x16_bf16.  These MFMAs run at 12 times the fp32 rate (1712
+// 8 significant bits, round to nearest), and a product is the six partial
+// products down to 2^-16 of it (h h, h m, m h, m m, h l, l h; what is left out
+// is below 2^-26), by v_mfma_f32_32x32x16_bf16.  bf16 has float32's exponents,
+// so the parts of an unscaled value below 2^-110 would underflow (relative
+// error 1e-6 at 2^-114, 2e-3 at 2^-125): both operands are split times 2^24,
+// which makes every part of every float32, denormals too, zero or a normal
+// bf16, and the sums are multiplied by 2^-48 at the end.  These MFMAs run at 12 times the fp32 rate (1712
 // against 142 TFLOP/s measured from registers), so six of them per product
 // leave a ceiling of 285 TFLOP/s.
 //
@@ -900,9 +903,9 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
 // x 4096 NT takes 190 us (fp32 MFMAs 250), 182 with one running sum, 157 with
 // nothing but the MFMAs.
 //
-// Infinities and values whose rounding to bf16 overflows do not split
-// (inf - inf): a tile whose sums are not all finite is computed again on the
-// fp32 MFMA, which gives what the fp32 kernels give.
+// Infinities, values from 2^104 and sums from 2^80 overflow here: a tile whose
+// sums are not all finite is computed again on the fp32 MFMA, which gives what
+// the fp32 kernels give.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -919,9 +922,11 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
 
-// values 2e, 2e + 1 of a chunk into its three planes
+constexpr float SB_SC = 0x1p24f, SB_UNSC = 0x1p-48f;  // of an operand, of a sum
+
+// values 2e, 2e + 1 of a chunk, times SB_SC, into its three planes
 __device__ __forceinline__ void split_pair(const float (&x)[8], int e, uintx4 (&o)[3], bool neg = false) {
-  const float a = neg ? -x[2 * e] : x[2 * e], b = neg ? -x[2 * e + 1] : x[2 * e + 1];
+  const float a = x[2 * e] * (neg ? -SB_SC : SB_SC), b = x[2 * e + 1] * (neg ? -SB_SC : SB_SC);
   const unsigned h = bf16_pair(a, b);
   const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
   const unsigned m = bf16_pair(ra, rb);
@@ -1085,7 +1090,10 @@ void gemm_split_bf16(GemmArgs p, int tiles_m, int tiles_n) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad = bad || !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+      for (int r = 0; r < 16; ++r) {
+        bad = bad || !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+        acc[i][j][r] *= SB_UNSC;
+      }
   if (__syncthreads_or(bad)) {  // the whole tile again in fp32, operands straight from memory
 #pragma unroll
     for (int i = 0; i < 2; ++i)

@@ -75,3 +75,33 @@ def test_gemm_split_values_beyond_the_split(dev):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
     assert np.all(np.abs(got[fin] - ref[fin]) <= 6 * K * 2.0 ** -24 * np.abs(ref[fin]))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+def test_gemm_split_small_and_large_values(dev, ta, tb):
+    """Rows of A and columns of B of any magnitude keep float32's relative
+    accuracy: bf16 parts of a value near the smallest float32 must not
+    underflow, nor do sums too large for the split lose their place.  Values
+    are scaled per row of op(A) and column of op(B) by 2^-145 .. 2^60 (no tile
+    overflows the split), in the last rows and columns by up to 2^120 (tiles
+    that do, with small rows among them); sums of denormals may round at each
+    of the K additions."""
+    M, N, K = 1604, 1540, 448
+    log(f"gemm small and large ta={ta} tb={tb}")
+    rng = np.random.default_rng(ta * 2 + tb)
+    ea, eb = rng.integers(-140, 61, size=(M, 1)), rng.integers(-140, 11, size=(1, N))
+    ea[0], ea[1] = -145, -126
+    ea[1280:], eb[:, 1280:] = rng.integers(-140, 121, size=(M - 1280, 1)), rng.integers(-140, 121, size=(1, N - 1280))
+    with np.errstate(under="ignore"):
+        a = np.ldexp(rng.normal(size=(M, K)), ea).astype(np.float32)
+        b = np.ldexp(rng.normal(size=(K, N)), np.where(rng.random((1, N)) < 0.5, eb, 0)).astype(np.float32)
+    got = _gemm(dev, ta, tb, np.ascontiguousarray(a.T) if ta else a, np.ascontiguousarray(b.T) if tb else b, M, N, K)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    ref, mag = a @ b, np.abs(a) @ np.abs(b)
+    fin = mag < np.finfo(np.float32).max  # no partial sum overflows
+    assert np.isfinite(got[fin]).all()
+    assert np.all(np.abs(got[fin] - ref[fin]) <= 6 * K * 2.0 ** -24 * mag[fin] + K * 2.0 ** -149)
+    tiny = fin & (mag < 2.0 ** -80) & (mag > 2.0 ** -100)
+    assert tiny.any()
+    err = (got[tiny] - ref[tiny]) / mag[tiny]
+    assert np.sqrt(np.mean(err * err)) <= 2.0 ** -24  # as for ordinary values: test_gemm_split's norm bound over sqrt(K)
