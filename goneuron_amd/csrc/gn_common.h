@@ -118,6 +118,9 @@ struct GemmArgs {
   int cs_rows, cs_cols;
   float cs_scale;
   int *cs_done;
+  // 1: a forward product (EPI_SCALE), or one that has to repeat its bits:
+  // fp32 MFMAs in their order of sums whatever the tiles
+  int fwd;
 };
 bool gemm_segments_ok(const GemmArgs &a);  // launch_gemm can take a's K segments
 

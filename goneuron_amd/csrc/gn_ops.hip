@@ -507,7 +507,7 @@ extern "C" int gn_lstm_seq_forward(gn_ctx *c, const float *x, const float *param
     GemmArgs g{};  // xw[b*T + t] = x_t . Wx_i (the input-gate rows, Q13)
     g.M = B * T; g.N = H; g.K = I;
     g.A = x; g.lda = I; g.B = Wx; g.ldb = I;
-    g.C = m.xw; g.ldc = H; g.alpha = 1.f;
+    g.C = m.xw; g.ldc = H; g.alpha = 1.f; g.fwd = 1;
     g.ws = c->scratch; g.ws_cap = c->scratch_floats;
     KTimer kt(c, GN_KCLASS_GEMM, "gemm_fwd", gemm_flops(g));
     HIP_OK(c, launch_gemm('N', 'T', EPI_SCALE, g, c->stream));
@@ -706,7 +706,7 @@ extern "C" int gn_swiglu_forward(gn_ctx *c, const float *x, const float *params,
     g.M = B; g.N = out2; g.K = in;
     g.A = x; g.lda = in;
     g.B = params; g.ldb = in;
-    g.C = work; g.ldc = out2; g.alpha = 1.0f;
+    g.C = work; g.ldc = out2; g.alpha = 1.0f; g.fwd = 1;
     g.ws = c->scratch; g.ws_cap = c->scratch_floats;
     KTimer kt(c, GN_KCLASS_GEMM, "gemm_fwd", gemm_flops(g));
     HIP_OK(c, launch_gemm('N', 'T', EPI_SCALE, g, c->stream));

@@ -2119,7 +2119,7 @@ static int model_forward(gn_model *M, const float *x, int B, bool for_loss) {
           g.M = B; g.N = out2; g.K = R.d.in_size;
           g.A = cur; g.lda = R.d.in_size;
           g.B = M->params + R.poff; g.ldb = R.d.in_size;
-          g.C = R.zbuf; g.ldc = out2; g.alpha = 1.0f;
+          g.C = R.zbuf; g.ldc = out2; g.alpha = 1.0f; g.fwd = 1;
           g.ws = c->scratch; g.ws_cap = c->scratch_floats;
           HIP_OK(c, launch_gemm('N', 'T', EPI_SCALE, g, c->stream));
         }
@@ -2209,7 +2209,7 @@ static int model_forward(gn_model *M, const float *x, int B, bool for_loss) {
           g.M = B * R.T; g.N = R.H; g.K = R.I;
           g.A = cur; g.lda = R.I;
           g.B = Wx; g.ldb = R.I;
-          g.C = R.xw; g.ldc = R.H; g.alpha = 1.0f;
+          g.C = R.xw; g.ldc = R.H; g.alpha = 1.0f; g.fwd = 1;
           g.ws = c->scratch; g.ws_cap = c->scratch_floats;
           HIP_OK(c, launch_gemm('N', 'T', EPI_SCALE, g, c->stream));
         }

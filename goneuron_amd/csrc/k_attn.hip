@@ -2378,8 +2378,9 @@ struct HeadOp {
   const float *p;
   bool scores;
 };
+// fwd: the forward's products and the backward's scores, which repeat them.
 hipError_t pair_gemm(char ta, char tb, int M, int N, int K, HeadOp A, HeadOp Bm, float *C, bool c_scores,
-                     int B, int T, int D, int NH, hipStream_t s) {
+                     int B, int T, int D, int NH, bool fwd, hipStream_t s) {
   const int hd = D / NH;
   const int64_t TT = (int64_t)T * T;
   GemmArgs a{};
@@ -2387,6 +2388,7 @@ hipError_t pair_gemm(char ta, char tb, int M, int N, int K, HeadOp A, HeadOp Bm,
   a.N = N;
   a.K = K;
   a.alpha = 1.f;
+  a.fwd = fwd;
   a.nbatch = B * NH;
   a.nbatch_in = NH;
   auto set = [&](HeadOp o, const float *&ptr, int &ld, int64_t &bs, int64_t &is) {
@@ -2429,9 +2431,9 @@ hipError_t launch_attn_fwd_any(const float *Q, const float *K, const float *V, f
   if (fa_supported(D, NH))
     return fa_run(Q, K, V, O, nullptr, nullptr, nullptr, nullptr, S, B, T, D, NH, causal, s);
   const int hd = D / NH;
-  hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, S, true, B, T, D, NH, s);
+  hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, S, true, B, T, D, NH, true, s);
   if (e == hipSuccess) e = softmax_scores(S, B, T, NH, hd, causal, s);
-  if (e == hipSuccess) e = pair_gemm('N', 'N', T, hd, T, {S, true}, {V, false}, O, false, B, T, D, NH, s);
+  if (e == hipSuccess) e = pair_gemm('N', 'N', T, hd, T, {S, true}, {V, false}, O, false, B, T, D, NH, true, s);
   return e;
 }
 
@@ -2442,18 +2444,18 @@ hipError_t launch_attn_bwd_any(const float *Q, const float *K, const float *V, c
     return fa_run(Q, K, V, const_cast<float *>(O), GO, GQ, GK, GV, S, B, T, D, NH, causal, s);
   const int hd = D / NH;
   float *P = S, *G = S + (size_t)B * NH * T * T;
-  hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, P, true, B, T, D, NH, s);
+  hipError_t e = pair_gemm('N', 'T', T, T, hd, {Q, false}, {K, false}, P, true, B, T, D, NH, true, s);
   if (e == hipSuccess) e = softmax_scores(P, B, T, NH, hd, causal, s);
-  if (e == hipSuccess) e = pair_gemm('N', 'T', T, T, hd, {GO, false}, {V, false}, G, true, B, T, D, NH, s);
+  if (e == hipSuccess) e = pair_gemm('N', 'T', T, T, hd, {GO, false}, {V, false}, G, true, B, T, D, NH, false, s);
   if (e == hipSuccess) {
     const int64_t rows = (int64_t)B * NH * T;
     hipLaunchKernelGGL(attn_dscore_rows, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, P, G, rows, T,
                        causal, (float)sqrt((double)hd));
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = pair_gemm('N', 'N', T, hd, T, {G, true}, {K, false}, GQ, false, B, T, D, NH, s);
-  if (e == hipSuccess) e = pair_gemm('T', 'N', T, hd, T, {G, true}, {Q, false}, GK, false, B, T, D, NH, s);
-  if (e == hipSuccess) e = pair_gemm('T', 'N', T, hd, T, {P, true}, {GO, false}, GV, false, B, T, D, NH, s);
+  if (e == hipSuccess) e = pair_gemm('N', 'N', T, hd, T, {G, true}, {K, false}, GQ, false, B, T, D, NH, false, s);
+  if (e == hipSuccess) e = pair_gemm('T', 'N', T, hd, T, {G, true}, {Q, false}, GK, false, B, T, D, NH, false, s);
+  if (e == hipSuccess) e = pair_gemm('T', 'N', T, hd, T, {P, true}, {GO, false}, GV, false, B, T, D, NH, false, s);
   return e;
 }
 

@@ -28,14 +28,15 @@
 // epilogue.
 //
 // 128-wide tiles whose K ranges are whole stages run a four-wave variant
-// instead (gemm_f32_mfma_w4) where they belong to a forward pass: one wave per
-// 64 x 64 sub-tile over the whole K range, operands fetched with direct global
-// -> LDS loads (no staging registers, no LDS store instructions), fragment
-// reads and loads issued one per MFMA.  With at least two tiles per CU it uses
+// instead (gemm_f32_mfma_w4) where they belong to a forward pass or add a
+// residual: one wave per 64 x 64 sub-tile over the whole K range, operands
+// fetched with direct global -> LDS loads (no staging registers, no LDS store
+// instructions), fragment reads and loads issued one per MFMA.  With at least two tiles per CU it uses
 // 32-deep stages so that two blocks share a CU and one block's prologue,
-// barriers and epilogue overlap the other's MFMAs.  Everywhere else those
-// tiles run on the bf16 matrix cores (gemm_split_bf16): each fp32 value as a
-// sum of three bf16, six partial products, an error below the fp32 MFMA's.
+// barriers and epilogue overlap the other's MFMAs.  Plain products and a
+// backward pass's dW and dX run those tiles on the bf16 matrix cores
+// (gemm_split_bf16): each fp32 value as a sum of three bf16, six partial
+// products, an error below the fp32 MFMA's.
 //
 // Used by Dense forward (NT: X[B,in] * W[out,in]^T, fused bias + activation),
 // Dense dX (NN: dZ[B,out] * W[out,in], fused activation derivative of the layer
@@ -1191,27 +1192,30 @@ template <int R, bool AK, bool BKC, int EPI>
 static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int tn, int splits,
                           int kchunk, hipStream_t s) {
   dim3 grid(tm * tn, splits, a.nbatch > 1 ? a.nbatch : 1), block(NT);
-  // 128-wide tiles over whole 64-deep K stages.  Plain products and those of
-  // the backward pass (C = alpha A B, dX with its activation derivative): the
-  // split-bf16 kernel (1024 x 4096 x 4096 NN 251 -> 202 us, 4096 x 4096 x 1024
-  // TN 261 -> 201, error 1.14e-6 -> 2.9e-7 and 5.7e-7 -> 1.5e-7).  A forward
-  // pass (bias, activation) keeps its order of fp32 sums: any other changes
-  // which units within rounding of 0 pass their ReLU, which moves a layer's
-  // gradient by 1e-3, where the split in the backward pass moves it by 1e-6.
-  // 64-wide tiles stay with eight waves of fp32 MFMAs, mostly faster there
-  // (4096 x 256 x 1024 22 against 28 us).
-  if constexpr (R == 128 && (EPI == EPI_SCALE || EPI == EPI_DACT)) {
+  if constexpr (R == 128) {
+    // 128-wide tiles over whole 64-deep K stages.  Plain products and those of
+    // the backward pass without an addend (C = alpha A B, dX with its
+    // activation derivative): the split-bf16 kernel (1024 x 4096 x 4096 NN 251
+    // -> 202 us, 4096 x 4096 x 1024 TN 261 -> 201, error 1.14e-6 -> 2.9e-7 and
+    // 5.7e-7 -> 1.5e-7).  A forward pass (bias and activation, or fwd) keeps
+    // its order of fp32 sums: any other changes which units within rounding of
+    // 0 pass their ReLU, which moves a layer's gradient by 1e-3, where the
+    // split in the backward pass moves it by 1e-6.  EPI_BIAS_ADD (the forward's
+    // residuals, the transformer's dX sums) stays on fp32 MFMAs too.  64-wide
+    // tiles stay with eight waves of fp32 MFMAs, mostly faster there
+    // (4096 x 256 x 1024 22 against 28 us).
+    constexpr bool split = EPI == EPI_SCALE || EPI == EPI_DACT;
     if (vec && !ktail) {
-      hipLaunchKernelGGL((gemm_split_bf16<AK, BKC, EPI>), grid, dim3(SB_NT), 0, s, a, tm, tn);
-      return hipGetLastError();
-    }
-  } else if constexpr (R == 128) {
-    // Four-wave kernels: 32-deep stages (64 KB of LDS) when there are at
-    // least two tiles per CU (two blocks share a CU) or the K range is at most
-    // four 64-deep stages (the transformer's K = 256 projections: +0.7 % on
-    // its step; at K = 1024 the C3 step lost 3 %); else 64-deep stages, one
-    // block per CU.
-    if (vec && !ktail) {
+      if constexpr (split)
+        if (!a.fwd) {
+          hipLaunchKernelGGL((gemm_split_bf16<AK, BKC, EPI>), grid, dim3(SB_NT), 0, s, a, tm, tn);
+          return hipGetLastError();
+        }
+      // Four-wave kernels: 32-deep stages (64 KB of LDS) when there are at
+      // least two tiles per CU (two blocks share a CU) or the K range is at most
+      // four 64-deep stages (the transformer's K = 256 projections: +0.7 % on
+      // its step; at K = 1024 the C3 step lost 3 %); else 64-deep stages, one
+      // block per CU.
       if (tm * tn >= 512 || kchunk <= 256)
         hipLaunchKernelGGL((gemm_f32_mfma_w4<32, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn, kchunk);
       else

@@ -105,3 +105,18 @@ def test_gemm_split_small_and_large_values(dev, ta, tb):
     assert tiny.any()
     err = (got[tiny] - ref[tiny]) / mag[tiny]
     assert np.sqrt(np.mean(err * err)) <= 2.0 ** -24  # as for ordinary values: test_gemm_split's norm bound over sqrt(K)
+
+
+def test_forward_products_keep_their_order_of_fp32_sums(dev):
+    """A forward product without bias (SwiGLU's [W x | V x]) has the bits of a
+    linear Dense layer of the same sizes with zero biases, in 128-wide tiles too."""
+    from goneuron_amd._lib import check, lib
+    B, I, O = 1604, 512, 800  # 13 x 13 tiles of 128
+    log("swiglu forward product")
+    rng = np.random.default_rng(3)
+    x, W = rng.normal(size=(B, I)).astype(np.float32), rng.normal(size=(2 * O, I)).astype(np.float32)
+    dx, dw, db = DBuf(dev, x), DBuf(dev, W), DBuf(dev, np.zeros(2 * O, np.float32))
+    z, out, work = (DBuf(dev, np.zeros(s, np.float32)) for s in ((B, 2 * O), (B, O), (4 * B, O)))
+    check(dev.h, lib().gn_dense_forward(dev.h, dx.p, dw.p, db.p, z.p, B, I, 2 * O, 6, 0))
+    check(dev.h, lib().gn_swiglu_forward(dev.h, dx.p, dw.p, out.p, work.p, B, I, O))
+    assert np.array_equal(work.get()[:2 * B].reshape(B, 2 * O), z.get())
