@@ -1204,10 +1204,14 @@ static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int 
     // residuals, the transformer's dX sums) stays on fp32 MFMAs too.  64-wide
     // tiles stay with eight waves of fp32 MFMAs, mostly faster there
     // (4096 x 256 x 1024 22 against 28 us).
+    // From five K stages on: four or fewer are bound by the operands' and C's
+    // traffic, and there the split only adds work (1664 x 1664 x 64 TN 10.3
+    // -> 11.3 us, 4096 x 4096 x 128 NT 54.5 -> 57.5; at K = 512 16384 x 512 x
+    // 512 is 73 -> 55).
     constexpr bool split = EPI == EPI_SCALE || EPI == EPI_DACT;
     if (vec && !ktail) {
       if constexpr (split)
-        if (!a.fwd) {
+        if (!a.fwd && a.K > 4 * BK) {
           hipLaunchKernelGGL((gemm_split_bf16<AK, BKC, EPI>), grid, dim3(SB_NT), 0, s, a, tm, tn);
           return hipGetLastError();
         }

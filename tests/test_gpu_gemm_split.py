@@ -46,6 +46,27 @@ def test_gemm_split(dev, ta, tb, M, N, K, pad):
         assert np.array_equal(got, (_op(A, ta).astype(np.float64) @ _op(B, tb)).astype(np.float32))
 
 
+@pytest.mark.parametrize("ta,tb,M,N,K,pad", [
+    (0, 1, 1601, 1543, 320, 0), (0, 1, 1536, 1792, 256, 0), (0, 0, 1601, 1540, 320, 8), (0, 0, 1537, 1668, 256, 0),
+    (1, 0, 1604, 1540, 320, 0), (1, 0, 1540, 1668, 256, 4), (1, 1, 1604, 1537, 320, 4), (1, 1, 1604, 1540, 256, 0),
+    (1, 0, 1604, 1540, 1088, 0)])
+def test_gemm_split_from_five_stages(dev, ta, tb, M, N, K, pad):
+    """The last K of the fp32 kernel and the first of the split, each order."""
+    test_gemm_split(dev, ta, tb, M, N, K, pad)
+
+
+def test_short_products_stay_on_fp32(dev):
+    """Up to K = 256 a plain product has the bits of a linear Dense forward."""
+    from goneuron_amd._lib import check, lib
+    B, I, O = 1604, 256, 1600
+    log("plain product of four K stages")
+    rng = np.random.default_rng(9)
+    x, W = rng.normal(size=(B, I)).astype(np.float32), rng.normal(size=(O, I)).astype(np.float32)
+    dx, dw, db, z = DBuf(dev, x), DBuf(dev, W), DBuf(dev, np.zeros(O, np.float32)), DBuf(dev, np.zeros((B, O), np.float32))
+    check(dev.h, lib().gn_dense_forward(dev.h, dx.p, dw.p, db.p, z.p, B, I, O, 6, 0))
+    assert np.array_equal(_gemm(dev, 0, 1, x, W, B, O, I), z.get())
+
+
 def test_gemm_split_has_no_bias(dev):
     M, N, K = 1536, 1792, 1024
     rng = np.random.default_rng(11)
