@@ -1859,19 +1859,21 @@ __device__ __forceinline__ float4 fa_load4(const float *__restrict__ p, int n) {
   return v;
 }
 
-// FULL (heads of exactly HD columns, 16-byte aligned): loads without guards,
-// rows past the end re-read the last one (their probabilities are 0 and their
-// results are not stored).  Otherwise columns past hd read as 0.
+// FULL: heads of exactly HD columns, 16-byte aligned.  Otherwise columns past
+// hd read as 0.  Rows past the end read as 0: their probabilities are 0, and 0
+// times an infinity of a re-read row would be NaN.
 
 // the lane's columns 16 x + 4*(l/16) .. +3 of row t
 template <int HD, bool FULL>
 __device__ __forceinline__ void fa_row(float4 (&v)[Fa<HD>::HX], const float *__restrict__ src, int t, int T, int D,
                                        int hd, int lane) {
   const int dl = 4 * (lane >> 4);
-  const float *p = src + (int64_t)min(t, T - 1) * D + dl;
+  const float *p = src + (int64_t)t * D + dl;
 #pragma unroll
-  for (int x = 0; x < Fa<HD>::HX; ++x)
-    v[x] = FULL ? *reinterpret_cast<const float4 *>(p + 16 * x) : fa_load4(p + 16 * x, hd - dl - 16 * x);
+  for (int x = 0; x < Fa<HD>::HX; ++x) {
+    if (FULL) v[x] = t < T ? *reinterpret_cast<const float4 *>(p + 16 * x) : make_float4(0.f, 0.f, 0.f, 0.f);
+    else v[x] = fa_load4(p + 16 * x, t < T ? hd - dl - 16 * x : 0);
+  }
 }
 
 // Staging of rows [k0, k0 + KS) of one matrix: thread t brings column group
@@ -1883,8 +1885,10 @@ __device__ __forceinline__ void fa_fetch(float4 (&v)[Fa<HD>::NL], const float *_
   const int r = k0 + (int)threadIdx.x / (HD / 4), c = 4 * (threadIdx.x % (HD / 4));
 #pragma unroll
   for (int q = 0; q < F::NL; ++q) {
-    const float *p = src + (int64_t)min(r + q * F::RP, T - 1) * D + c;
-    v[q] = FULL ? *reinterpret_cast<const float4 *>(p) : fa_load4(p, hd - c);
+    const int t = r + q * F::RP;
+    const float *p = src + (int64_t)t * D + c;
+    if (FULL) v[q] = t < T ? *reinterpret_cast<const float4 *>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
+    else v[q] = fa_load4(p, t < T ? hd - c : 0);
   }
 }
 template <int HD>

@@ -75,3 +75,22 @@ def test_attn_single_key_rows_have_no_score_gradient(dev):
         _, got, _ = _mha(dev, 3, T, D, NH, 1, p, x, g)
         assert not got[:2 * (D * D + D)].any(), (T, D, NH)
         assert got[2 * (D * D + D):].any()
+
+
+def test_attn_infinite_last_row(dev):
+    """Positions past the end weigh nothing: an infinite value (or output
+    gradient) of the last token gives infinities, not NaN, in what it reaches."""
+    for T, D, NH in ((130, 64, 2), (33, 48, 1), (100, 128, 1), (70, 80, 2), (131, 24, 3)):
+        log(f"attention with an infinite last row T={T} D={D} heads={NH}")
+        rng = np.random.default_rng(T)
+        w = [np.zeros((D + 1, D), np.float32) for _ in range(4)]
+        w[0][:D], w[1][:D] = (rng.normal(size=(D, D)) * 1e-31 for _ in range(2))
+        w[2][:D] = 1e10  # V and gO of a token of 1e30 overflow, its Q and K do not
+        w[3][:D] = 1e10
+        p = np.concatenate([m.ravel() for m in w])
+        x = np.abs(rng.normal(size=(2, T, D))).astype(np.float32) * 1e-12
+        g = x.copy()
+        x[:, -1], g[:, -1] = 1e30, 1e30
+        out, gr, _ = _mha(dev, 2, T, D, NH, 0, p, x.reshape(2, T * D), g.reshape(2, T * D))
+        assert np.all(out == np.inf), (T, D)
+        assert np.all(gr[3 * (D * D + D) - D:3 * (D * D + D)] == np.inf), (T, D)  # V's bias gradient
