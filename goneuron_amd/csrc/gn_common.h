@@ -569,8 +569,9 @@ bool attn_supported(int T, int D, int NH);  // the fused kernels: T <= 128, D / 
 // Attention of any T and head size: heads of up to 128 in kernels that stage
 // the other side's rows, wider ones through batched GEMMs over the (sample,
 // head) pairs and row kernels.  `S` (attn_work_floats) carries what the
-// forward leaves for the backward: (maximum, 1 / sum) per row, or the
-// materialised scores and their gradients.  O: the forward's output.
+// forward leaves for the backward, (maximum, 1 / sum) per row, and the
+// backward's row sums, or the materialised scores and their gradients.  O: the
+// forward's output.
 size_t attn_work_floats(int B, int T, int D, int NH);
 hipError_t launch_attn_fwd_any(const float *Q, const float *K, const float *V, float *O, int B, int T,
                                int D, int NH, int causal, float *S, hipStream_t s);

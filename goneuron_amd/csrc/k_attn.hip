@@ -1821,23 +1821,25 @@ bool attn_supported(int T, int D, int NH) {
 constexpr int FA_B = 64;    // rows per workgroup (16 per wave) where they fill the chip
 constexpr int FA_NT = 256;
 
-// exp of a float32 argument <= 0 in float32: x = n ln 2 + r with n ln2_hi
-// exact, the Taylor polynomial of degree 7 in |r| <= ln 2 / 2 and one rounding
-// at the end: 1.03 ulp at most, 0.31 rms (float64 exp rounded to float32: 0.5
-// and 0.29; in float64 the exponentials took as long as the products around
-// them).  NaN in,
-// NaN out; below -104 the float32 result is 0.
+// float32(exp(x)) for x <= 0 in float64 after Cody and Waite's reduction x = n
+// ln 2 + r: the Taylor polynomial of degree 9 in |r| <= ln 2 / 2 is within
+// 7e-12, so the float32 result differs from the float64 exponential's rounding
+// in one of 200,000 arguments (0.5001 ulp at most), at a third of the library
+// exp's instructions.  NaN in, NaN out; below -104 the result is 0.
 __device__ __forceinline__ float exp32(float x) {
   const float c = x < -104.0f ? -104.0f : x;
   const float n = __builtin_rintf(c * 1.44269504f);
-  float r = __builtin_fmaf(n, -0.693145752f, c);
-  r = __builtin_fmaf(n, -1.42860677e-06f, r);
-  float p = __builtin_fmaf(1.0f / 5040.0f, r, 1.0f / 720.0f);
-  p = __builtin_fmaf(p, r, 1.0f / 120.0f);
-  p = __builtin_fmaf(p, r, 1.0f / 24.0f);
-  p = __builtin_fmaf(p, r, 1.0f / 6.0f);
-  p = __builtin_fmaf(p, r, 0.5f);
-  return __builtin_ldexpf(1.0f + __builtin_fmaf(p, r * r, r), (int)n);
+  const double r = __builtin_fma((double)n, -0.6931471805599453, (double)c);
+  double p = __builtin_fma(1.0 / 362880.0, r, 1.0 / 40320.0);
+  p = __builtin_fma(p, r, 1.0 / 5040.0);
+  p = __builtin_fma(p, r, 1.0 / 720.0);
+  p = __builtin_fma(p, r, 1.0 / 120.0);
+  p = __builtin_fma(p, r, 1.0 / 24.0);
+  p = __builtin_fma(p, r, 1.0 / 6.0);
+  p = __builtin_fma(p, r, 0.5);
+  p = __builtin_fma(p, r, 1.0);
+  p = __builtin_fma(p, r, 1.0);
+  return __builtin_ldexpf((float)p, (int)n);
 }
 
 template <int HD>
@@ -1929,6 +1931,12 @@ __device__ __forceinline__ void fa_acc(fx4 (&o)[Fa<HD>::HX], const float *sy, co
     for (int x = 0; x < Fa<HD>::HX; ++x) o[x] = mfma16(p[s * Fa<HD>::P + 16 * x], zt[s], o[x]);
 }
 
+template <int HD>
+__device__ __forceinline__ void fa_zero(fx4 (&o)[Fa<HD>::HX]) {
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x) o[x] = fx4{0.f, 0.f, 0.f, 0.f};
+}
+
 template <int HD, bool FULL>
 __device__ __forceinline__ void fa_store(float *__restrict__ G, const fx4 (&o)[Fa<HD>::HX], int64_t base, int t, int T,
                                          int D, int hd, int lane) {
@@ -1980,29 +1988,6 @@ __device__ __forceinline__ void fa_merge(fx4 (&o)[Fa<HD>::HX], float *buf) {
   }
 }
 
-// The diagonal of a 16 x 16 product tile: element (i, i) of lane column i.
-__device__ __forceinline__ float fa_diag(const fx4 &t, int lane) {
-  const int i = lane & 15;
-  const float v = (i & 3) == 0 ? t[0] : (i & 3) == 1 ? t[1] : (i & 3) == 2 ? t[2] : t[3];
-  return fa_sum4((lane >> 4) == (i >> 2) ? v : 0.f);
-}
-
-// d_i = gO_i . o_i through the instructions, and in the order, that form dP_ij
-// = gO_i . v_j: where a row has one key (o_i = v_j, P = 1) dP - d is then an
-// exact zero, as in the reference's sum over the row.
-template <int HD>
-__device__ __forceinline__ float fa_rowdot(const float4 (&o)[Fa<HD>::HX], const float4 (&g)[Fa<HD>::HX], int lane) {
-  fx4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
-#pragma unroll
-  for (int x = 0; x < Fa<HD>::HX; ++x) {
-    a0 = mfma16(o[x].x, g[x].x, a0);
-    a1 = mfma16(o[x].y, g[x].y, a1);
-    a0 = mfma16(o[x].z, g[x].z, a0);
-    a1 = mfma16(o[x].w, g[x].w, a1);
-  }
-  return fa_diag(a0 + a1, lane);
-}
-
 // Block -> (pair, row block): the blocks of a pair are `npair` apart, so with
 // a multiple of 8 pairs they run on one XCD and share its L2; under the causal
 // mask the longest blocks are dispatched first.
@@ -2027,8 +2012,7 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
   float4 qr[F::HX];
   fa_row<HD, FULL>(qr, Q + base, qi, T, D, hd, lane);
   fx4 o[F::HX];
-#pragma unroll
-  for (int x = 0; x < F::HX; ++x) o[x] = fx4{0.f, 0.f, 0.f, 0.f};
+  fa_zero<HD>(o);
   float m = -__builtin_inff(), l = 0.f;  // running maximum; the lane's own part of the sum
   const int kend = causal ? min(T, qb * RB + RB) : T;
   float4 kv[F::NL], vv[F::NL];
@@ -2068,19 +2052,22 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
       const float mn = fmaxf(m, fa_max4(mx));
       const float ms = mn == -__builtin_inff() ? 0.f : mn;  // only -inf so far: weights 0
       const float al = exp32(m - ms);
-      l *= al;
-#pragma unroll
-      for (int x = 0; x < F::HX; ++x) o[x] = o[x] * al;
+      fx4 os[F::HX];  // the stage's own sums
+      float ls = 0.f;
+      fa_zero<HD>(os);
 #pragma unroll
       for (int kt = 0; kt < F::KS / 16; ++kt) {
         if (!mine(kt)) continue;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[kt][r] = exp32(s[kt][r] - ms);
-          l += s[kt][r];
-        }
-        fa_acc<HD>(o, sv, s[kt], kt, lane);
+        for (int r = 0; r < 4; ++r) s[kt][r] = exp32(s[kt][r] - ms);
+        ls += (s[kt][0] + s[kt][1]) + (s[kt][2] + s[kt][3]);
+        fa_acc<HD>(os, sv, s[kt], kt, lane);
       }
+      l = __builtin_fmaf(l, al, ls);
+#pragma unroll
+      for (int x = 0; x < F::HX; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[x][r] = __builtin_fmaf(o[x][r], al, os[x][r]);
       m = mn;
     }
     __syncthreads();
@@ -2106,165 +2093,237 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
   if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = make_float2(m, il);
 }
 
+// c_i = gO_i . o_i (the lane's row) through the instructions, and in the order,
+// that form dP_ij = gO_i . v_j: the diagonal of a 16 x 16 product tile.
+template <int HD>
+__device__ __forceinline__ float fa_rowdot(const float4 (&o)[Fa<HD>::HX], const float4 (&g)[Fa<HD>::HX], int lane) {
+  fx4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+  for (int x = 0; x < Fa<HD>::HX; ++x) {
+    a0 = mfma16(o[x].x, g[x].x, a0);
+    a1 = mfma16(o[x].y, g[x].y, a1);
+    a0 = mfma16(o[x].z, g[x].z, a0);
+    a1 = mfma16(o[x].w, g[x].w, a1);
+  }
+  const fx4 t = a0 + a1;
+  const int i = lane & 15;
+  const float v = (i & 3) == 0 ? t[0] : (i & 3) == 1 ? t[1] : (i & 3) == 2 ? t[2] : t[3];
+  return fa_sum4((lane >> 4) == (i >> 2) ? v : 0.f);
+}
+
 // Backward: gradScore = P (dP - d) / sqrt(hd), dP_ij = gO_i . v_j, d_i =
-// sum_j P_ij dP_ij = gO_i . o_i.  Two roles in one launch, each recomputing P
-// from the saved (maximum, 1 / sum), so every result has one writer and one
-// order of sums: key blocks (gK, gV over the live queries), dispatched first
-// as they do four products per tile pair, and query blocks (gQ over the live
-// keys, three products).
+// sum_j P_ij dP_ij.  Both kernels recompute P from the saved (maximum, 1 /
+// sum), so every result has one writer and one order of sums.  Query blocks
+// (three products per tile pair) come first.  They take d_i = gO_i . o_i,
+// equal to the sum but for the rounding of o and dP, which is below that of
+// gQ; it would stay, though, in the key blocks' sums over keys, which vanish
+// but for it (the key projection's error against float64 was 1.2 to 2.8 times
+// that of the sum).  So the query blocks also sum P (dP - d), the difference,
+// and leave the key blocks d with it: where a row has one key, P = 1, dP - d is
+// then an exact zero, as in the reference.  A row of one stage of keys, where
+// few probabilities average that rounding, has the sum before its gQ and takes
+// it there too.
 template <int HD, bool SP, bool FULL>
-__global__ __launch_bounds__(FA_NT) void fa_bwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
-                                                       const float *__restrict__ V, const float *__restrict__ O,
-                                                       const float *__restrict__ GO, float *__restrict__ GQ,
-                                                       float *__restrict__ GK, float *__restrict__ GV,
-                                                       const float2 *__restrict__ st, int T, int D, int NH, int hd,
-                                                       int causal, int npair, int nb) {
+__global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K,
+                                                         const float *__restrict__ V, const float *__restrict__ O,
+                                                         const float *__restrict__ GO, float *__restrict__ GQ,
+                                                         const float2 *__restrict__ st, float *__restrict__ dr, int T,
+                                                         int D, int NH, int hd, int causal, int npair, int nb) {
+  using F = Fa<HD>;
+  constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
+  __shared__ __align__(16) float sh[2 * F::KS * F::P];
+  __shared__ float sd[4][16];
+  float *sa = sh, *sb = sh + F::KS * F::P;  // K rows, V rows
+  const int pair = blockIdx.x % npair, rb = nb - 1 - blockIdx.x / npair;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, dl = 4 * (lane >> 4);
+  const int64_t base = (int64_t)(pair / NH) * T * D + (pair % NH) * hd;
+  const float is = 1.0f / (float)sqrt((double)hd);
+  const int r0 = rb * RB + (SP ? 0 : 16 * w), ri = r0 + (lane & 15);  // the wave's and the lane's row
+  float4 av[F::NL], bv[F::NL], za[F::HX], zb[F::HX];
+  fx4 ga[F::HX];
+  fa_zero<HD>(ga);
+  fa_row<HD, FULL>(za, O + base, ri, T, D, hd, lane);
+  fa_row<HD, FULL>(zb, GO + base, ri, T, D, hd, lane);
+  const float c = fa_rowdot<HD>(za, zb, lane);
+  fa_row<HD, FULL>(za, Q + base, ri, T, D, hd, lane);
+  const float2 ml = ri < T ? st[(int64_t)pair * T + ri] : make_float2(0.f, 0.f);
+  const int kend = causal ? min(T, rb * RB + RB) : T;
+  float dsum = 0.f;  // of P (dP - c)
+  auto row_sum = [&](float v) {  // over the lane groups and, with SP, the waves
+    v = fa_sum4(v);
+    if (!SP) return v;
+    if (lane < 16) sd[w][lane] = v;
+    __syncthreads();
+    const int i = lane & 15;
+    return (sd[0][i] + sd[1][i]) + (sd[2][i] + sd[3][i]);
+  };
+  const bool one = kend <= F::KS;  // uniform over the workgroup
+  fa_fetch<HD, FULL>(av, K + base, 0, T, D, hd);
+  fa_fetch<HD, FULL>(bv, V + base, 0, T, D, hd);
+  for (int k0 = 0; k0 < kend; k0 += F::KS) {
+    fa_put<HD>(sa, av);
+    fa_put<HD>(sb, bv);
+    __syncthreads();
+    if (k0 + F::KS < kend) {
+      fa_fetch<HD, FULL>(av, K + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, FULL>(bv, V + base, k0 + F::KS, T, D, hd);
+    }
+    if (r0 < T) {
+      auto mine = [&](int kt) {  // uniform over the wave
+        const int jb = k0 + 16 * kt;
+        return jb < T && !(causal && jb > r0 + 15) && (!SP || ((jb >> 4) & 3) == w);
+      };
+      fx4 ps[KT], ds[KT];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        if (!mine(kt)) continue;
+        const int jb = k0 + 16 * kt;
+        const fx4 s = fa_tile<HD>(sa, za, kt, lane), dp = fa_tile<HD>(sb, zb, kt, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          ps[kt][r] = exp32(s[r] * is - ml.x) * ml.y;
+          ds[kt][r] = ps[kt][r] * (dp[r] - c);
+        }
+        if (jb + 15 >= T || r0 + 15 >= T || (causal && jb + 15 > r0)) {  // uniform: a tile at an edge
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = jb + dl + r;
+            const bool live = j < T && ri < T && !(causal && j > ri);
+            ps[kt][r] = live ? ps[kt][r] : 0.f;
+            ds[kt][r] = live ? ds[kt][r] : 0.f;
+          }
+        }
+        dsum += (ds[kt][0] + ds[kt][1]) + (ds[kt][2] + ds[kt][3]);
+      }
+      if (one) dsum = row_sum(dsum);
+      fx4 gs[F::HX];  // the stage's own sums
+      fa_zero<HD>(gs);
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        if (!mine(kt)) continue;
+        if (one) ds[kt] = ds[kt] - ps[kt] * dsum;
+        fa_acc<HD>(gs, sa, ds[kt] * is, kt, lane);  // gQ_i += gradScore_ij k_j
+      }
+#pragma unroll
+      for (int x = 0; x < F::HX; ++x) ga[x] = ga[x] + gs[x];
+    }
+    __syncthreads();
+  }
+  if (!one) dsum = row_sum(dsum);
+  if (SP) {
+    fa_merge<HD>(ga, sh);
+    if (w > 0) return;
+  }
+  if (lane < 16 && ri < T) dr[(int64_t)pair * T + ri] = c + dsum;
+  fa_store<HD, FULL>(GQ, ga, base, ri, T, D, hd, lane);
+}
+
+// Key blocks: gK and gV over the live queries, four products per tile pair.
+template <int HD, bool SP, bool FULL>
+__global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict__ Q, const float *__restrict__ K,
+                                                         const float *__restrict__ V, const float *__restrict__ GO,
+                                                         float *__restrict__ GK, float *__restrict__ GV,
+                                                         const float2 *__restrict__ st, const float *__restrict__ dr,
+                                                         int T, int D, int NH, int hd, int causal, int npair, int nb) {
   using F = Fa<HD>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
   __shared__ __align__(16) float sm[F::KS], sl[F::KS], sd[F::KS];
-  float *sa = sh;                   // keys: K rows; queries: Q rows
-  float *sb = sh + F::KS * F::P;    // keys: V rows; queries: gO rows
-  const bool kside = (int)blockIdx.x < npair * nb;
-  const int bid = kside ? blockIdx.x : blockIdx.x - npair * nb;
-  const int pair = bid % npair, rb = kside ? bid / npair : nb - 1 - bid / npair;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, tid = threadIdx.x;
-  const int dl = 4 * (lane >> 4);
+  float *sa = sh, *sb = sh + F::KS * F::P;  // Q rows, gO rows
+  const int pair = blockIdx.x % npair, rb = blockIdx.x / npair;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, dl = 4 * (lane >> 4);
   const int64_t base = (int64_t)(pair / NH) * T * D + (pair % NH) * hd;
   const float is = 1.0f / (float)sqrt((double)hd);
   const int r0 = rb * RB + (SP ? 0 : 16 * w), ri = r0 + (lane & 15);  // the wave's and the lane's row
   const float2 *stp = st + (int64_t)pair * T;
-  float4 av[F::NL], bv[F::NL];
-  float4 za[F::HX], zb[F::HX], ov[F::HX];
+  const float *dp0 = dr + (int64_t)pair * T;
+  float4 av[F::NL], bv[F::NL], za[F::HX], zb[F::HX];
   fx4 ga[F::HX], gb[F::HX];
+  fa_zero<HD>(ga);
+  fa_zero<HD>(gb);
+  fa_row<HD, FULL>(za, K + base, ri, T, D, hd, lane);
+  fa_row<HD, FULL>(zb, V + base, ri, T, D, hd, lane);
+  const int i0 = causal ? rb * RB / F::KS * F::KS : 0;  // first stage with a live query
+  // the saved statistics and d of a stage's queries: wave w its tile w
+  float2 ml;
+  float dq;
+  auto fetch_rows = [&](int k0) {
+    const int t = k0 + 16 * w + lane;
+    if (w >= KT || lane >= 16) return;
+    ml = t < T ? stp[t] : make_float2(0.f, 0.f);  // rows past the end: probability 0
+    dq = t < T ? dp0[t] : 0.f;
+  };
+  fa_fetch<HD, FULL>(av, Q + base, i0, T, D, hd);
+  fa_fetch<HD, FULL>(bv, GO + base, i0, T, D, hd);
+  fetch_rows(i0);
+  for (int k0 = i0; k0 < T; k0 += F::KS) {
+    fa_put<HD>(sa, av);
+    fa_put<HD>(sb, bv);
+    if (w < KT && lane < 16) {
+      sm[16 * w + lane] = ml.x;
+      sl[16 * w + lane] = ml.y;
+      sd[16 * w + lane] = dq;
+    }
+    __syncthreads();
+    if (k0 + F::KS < T) {
+      fa_fetch<HD, FULL>(av, Q + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, FULL>(bv, GO + base, k0 + F::KS, T, D, hd);
+      fetch_rows(k0 + F::KS);
+    }
+    if (r0 < T) {
+      fx4 gas[F::HX], gbs[F::HX];  // the stage's own sums
+      fa_zero<HD>(gas);
+      fa_zero<HD>(gbs);
 #pragma unroll
-  for (int x = 0; x < F::HX; ++x) ga[x] = gb[x] = fx4{0.f, 0.f, 0.f, 0.f};
-  if (kside) {
-    fa_row<HD, FULL>(za, K + base, ri, T, D, hd, lane);
-    fa_row<HD, FULL>(zb, V + base, ri, T, D, hd, lane);
-    const int i0 = causal ? rb * RB / F::KS * F::KS : 0;  // first stage with a live query
-    // d and the saved statistics of a stage's queries: wave w its tile w
-    float2 ml;
-    auto fetch_rows = [&](int k0) {
-      if (w >= KT) return;
-      const int t = k0 + 16 * w + (lane & 15);
-      fa_row<HD, FULL>(ov, O + base, t, T, D, hd, lane);
-      ml = t < T ? stp[t] : make_float2(0.f, 0.f);  // rows past the end: probability 0
-    };
-    fa_fetch<HD, FULL>(av, Q + base, i0, T, D, hd);
-    fa_fetch<HD, FULL>(bv, GO + base, i0, T, D, hd);
-    fetch_rows(i0);
-    for (int k0 = i0; k0 < T; k0 += F::KS) {
-      fa_put<HD>(sa, av);
-      fa_put<HD>(sb, bv);
-      __syncthreads();
-      if (w < KT) {
-        float4 gr[F::HX];
-        const float4 *p = reinterpret_cast<const float4 *>(sb + (16 * w + (lane & 15)) * F::P + dl);
+      for (int qt = 0; qt < KT; ++qt) {
+        const int ib = k0 + 16 * qt;
+        if (ib >= T || (causal && ib + 15 < r0) || (SP && ((ib >> 4) & 3) != w)) continue;  // uniform over the wave
+        fx4 s = fa_tile<HD>(sa, za, qt, lane), dp = fa_tile<HD>(sb, zb, qt, lane);
+        const float4 m4 = *reinterpret_cast<const float4 *>(sm + 16 * qt + dl);
+        const float4 l4 = *reinterpret_cast<const float4 *>(sl + 16 * qt + dl);
+        const float4 d4 = *reinterpret_cast<const float4 *>(sd + 16 * qt + dl);
+        const float mm[4] = {m4.x, m4.y, m4.z, m4.w}, ll[4] = {l4.x, l4.y, l4.z, l4.w};
+        const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+        fx4 ds;
 #pragma unroll
-        for (int x = 0; x < F::HX; ++x) gr[x] = p[4 * x];
-        const float d = fa_rowdot<HD>(ov, gr, lane);
-        if (lane < 16) {
-          sm[16 * w + lane] = ml.x;
-          sl[16 * w + lane] = ml.y;
-          sd[16 * w + lane] = d;
+        for (int r = 0; r < 4; ++r) {
+          s[r] = exp32(s[r] * is - mm[r]) * ll[r];
+          ds[r] = s[r] * (dp[r] - dd[r]) * is;
         }
-      }
-      if (k0 + F::KS < T) {
-        fa_fetch<HD, FULL>(av, Q + base, k0 + F::KS, T, D, hd);
-        fa_fetch<HD, FULL>(bv, GO + base, k0 + F::KS, T, D, hd);
-        fetch_rows(k0 + F::KS);
-      }
-      __syncthreads();
-      if (r0 < T) {
-#pragma unroll
-        for (int qt = 0; qt < KT; ++qt) {
-          const int ib = k0 + 16 * qt;
-          if (ib >= T || (causal && ib + 15 < r0) || (SP && ((ib >> 4) & 3) != w)) continue;  // uniform over the wave
-          fx4 s = fa_tile<HD>(sa, za, qt, lane), dp = fa_tile<HD>(sb, zb, qt, lane);
-          const float4 m4 = *reinterpret_cast<const float4 *>(sm + 16 * qt + dl);
-          const float4 l4 = *reinterpret_cast<const float4 *>(sl + 16 * qt + dl);
-          const float4 d4 = *reinterpret_cast<const float4 *>(sd + 16 * qt + dl);
-          const float mm[4] = {m4.x, m4.y, m4.z, m4.w}, ll[4] = {l4.x, l4.y, l4.z, l4.w};
-          const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
-          fx4 ds;
+        if (ib + 15 >= T || r0 + 15 >= T || (causal && r0 + 15 > ib)) {  // uniform: a tile at an edge
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            s[r] = exp32(s[r] * is - mm[r]) * ll[r];
-            ds[r] = s[r] * (dp[r] - dd[r]) * is;
+            const int i = ib + dl + r;
+            const bool live = i < T && ri < T && !(causal && ri > i);
+            s[r] = live ? s[r] : 0.f;
+            ds[r] = live ? ds[r] : 0.f;
           }
-          if (ib + 15 >= T || r0 + 15 >= T || (causal && r0 + 15 > ib)) {  // uniform: a tile at an edge
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int i = ib + dl + r;
-              const bool live = i < T && ri < T && !(causal && ri > i);
-              s[r] = live ? s[r] : 0.f;
-              ds[r] = live ? ds[r] : 0.f;
-            }
-          }
-          fa_acc<HD>(gb, sb, s, qt, lane);   // gV_j += p_ij gO_i
-          fa_acc<HD>(ga, sa, ds, qt, lane);  // gK_j += gradScore_ij q_i
         }
+        fa_acc<HD>(gbs, sb, s, qt, lane);   // gV_j += p_ij gO_i
+        fa_acc<HD>(gas, sa, ds, qt, lane);  // gK_j += gradScore_ij q_i
       }
-      __syncthreads();
-    }
-    if (SP) {
-      fa_merge<HD>(ga, sh);
-      fa_merge<HD>(gb, sh);
-      if (w > 0) return;
-    }
-    fa_store<HD, FULL>(GK, ga, base, ri, T, D, hd, lane);
-    fa_store<HD, FULL>(GV, gb, base, ri, T, D, hd, lane);
-  } else {
-    fa_row<HD, FULL>(za, Q + base, ri, T, D, hd, lane);
-    fa_row<HD, FULL>(zb, GO + base, ri, T, D, hd, lane);
-    fa_row<HD, FULL>(ov, O + base, ri, T, D, hd, lane);
-    const float dsum = fa_rowdot<HD>(ov, zb, lane);
-    const float2 ml = ri < T ? stp[ri] : make_float2(0.f, 0.f);
-    const int kend = causal ? min(T, rb * RB + RB) : T;
-    fa_fetch<HD, FULL>(av, K + base, 0, T, D, hd);
-    fa_fetch<HD, FULL>(bv, V + base, 0, T, D, hd);
-    for (int k0 = 0; k0 < kend; k0 += F::KS) {
-      fa_put<HD>(sa, av);
-      fa_put<HD>(sb, bv);
-      __syncthreads();
-      if (k0 + F::KS < kend) {
-        fa_fetch<HD, FULL>(av, K + base, k0 + F::KS, T, D, hd);
-        fa_fetch<HD, FULL>(bv, V + base, k0 + F::KS, T, D, hd);
+#pragma unroll
+      for (int x = 0; x < F::HX; ++x) {
+        ga[x] = ga[x] + gas[x];
+        gb[x] = gb[x] + gbs[x];
       }
-      if (r0 < T) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-          const int jb = k0 + 16 * kt;
-          if (jb >= T || (causal && jb > r0 + 15) || (SP && ((jb >> 4) & 3) != w)) continue;
-          const fx4 s = fa_tile<HD>(sa, za, kt, lane), dp = fa_tile<HD>(sb, zb, kt, lane);
-          fx4 ds;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ds[r] = exp32(s[r] * is - ml.x) * ml.y * (dp[r] - dsum) * is;
-          if (jb + 15 >= T || r0 + 15 >= T || (causal && jb + 15 > r0)) {  // uniform: a tile at an edge
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int j = jb + dl + r;
-              ds[r] = j < T && ri < T && !(causal && j > ri) ? ds[r] : 0.f;
-            }
-          }
-          fa_acc<HD>(ga, sa, ds, kt, lane);  // gQ_i += gradScore_ij k_j
-        }
-      }
-      __syncthreads();
     }
-    if (SP) {
-      fa_merge<HD>(ga, sh);
-      if (w > 0) return;
-    }
-    fa_store<HD, FULL>(GQ, ga, base, ri, T, D, hd, lane);
+    __syncthreads();
   }
+  if (SP) {
+    fa_merge<HD>(ga, sh);
+    fa_merge<HD>(gb, sh);
+    if (w > 0) return;
+  }
+  fa_store<HD, FULL>(GK, ga, base, ri, T, D, hd, lane);
+  fa_store<HD, FULL>(GV, gb, base, ri, T, D, hd, lane);
 }
 
 static bool fa_supported(int D, int NH) { return NH > 0 && D % NH == 0 && D / NH <= 128; }
 
 size_t attn_work_floats(int B, int T, int D, int NH) {
-  return 2 * (size_t)B * NH * T * (fa_supported(D, NH) ? 1 : T);
+  const size_t rows = (size_t)B * NH * T;
+  return fa_supported(D, NH) ? 3 * rows : 2 * rows * T;  // (maximum, 1 / sum) and d; scores and their gradients
 }
 
 template <int HD, bool SP, bool FULL>
@@ -2274,12 +2333,19 @@ static hipError_t fa_launch(const float *Q, const float *K, const float *V, floa
   const int64_t np = (int64_t)B * NH;
   if (np * nb * 2 > 0x7fffffff) return hipErrorInvalidValue;
   float2 *st = reinterpret_cast<float2 *>(S);
-  if (!GO)
-    hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, FULL>), dim3((unsigned)(np * nb)), dim3(FA_NT), 0, s, Q, K, V, O, st, T,
-                       D, NH, hd, causal, (int)np, nb);
-  else
-    hipLaunchKernelGGL((fa_bwd_kernel<HD, SP, FULL>), dim3((unsigned)(2 * np * nb)), dim3(FA_NT), 0, s, Q, K, V, O, GO,
-                       GQ, GK, GV, st, T, D, NH, hd, causal, (int)np, nb);
+  float *dr = S + 2 * np * T;
+  const dim3 grid((unsigned)(np * nb)), block(FA_NT);
+  if (!GO) {
+    hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, O, st, T, D, NH, hd, causal, (int)np,
+                       nb);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((fa_bwd_q_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, O, GO, GQ, st, dr, T, D, NH, hd,
+                     causal, (int)np, nb);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fa_bwd_k_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, GO, GK, GV, st, dr, T, D, NH, hd,
+                     causal, (int)np, nb);
   return hipGetLastError();
 }
 

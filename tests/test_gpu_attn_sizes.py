@@ -94,3 +94,37 @@ def test_attn_infinite_last_row(dev):
         out, gr, _ = _mha(dev, 2, T, D, NH, 0, p, x.reshape(2, T * D), g.reshape(2, T * D))
         assert np.all(out == np.inf), (T, D)
         assert np.all(gr[3 * (D * D + D) - D:3 * (D * D + D)] == np.inf), (T, D)  # V's bias gradient
+
+
+@pytest.mark.parametrize("T,D,NH,causal", [(486, 48, 3, 0), (112, 128, 1, 1), (38, 64, 1, 1), (300, 128, 2, 1), (197, 192, 3, 0)])
+def test_attn_vanishing_sums(dev, T, D, NH, causal):
+    """Without rotary embedding the key projection's bias gradient vanishes:
+    every row of gradScore sums to zero.  What is left is the rounding of P, dP
+    and their row sums, which must not exceed that of float32 arithmetic in the
+    reference's order of operations (float64 exponential, d = sum P dP): here
+    numpy's, with half as much again allowed for one draw of 4 samples."""
+    B, hd = 4, D // NH
+    log(f"attention vanishing sums T={T} D={D} heads={NH} causal={causal}")
+    rng = np.random.default_rng(T + D)
+    p = (rng.normal(size=4 * (D * D + D)) / np.sqrt(D)).astype(np.float32)
+    x, g = (rng.normal(size=(B, T, D)).astype(np.float32) for _ in range(2))
+    _, got, _ = _mha(dev, B, T, D, NH, causal, p, x.reshape(B, -1), g.reshape(B, -1))
+    n1 = D * D + D
+    w = [(p[i * n1:i * n1 + D * D].reshape(D, D), p[i * n1 + D * D:(i + 1) * n1]) for i in range(4)]
+    q, k, v = (x @ w[i][0].T + w[i][1] for i in range(3))
+    go = g @ w[3][0]
+    left = np.zeros(D, np.float32)
+    mask = np.triu(np.ones((T, T), bool), 1) if causal else np.zeros((T, T), bool)
+    for b in range(B):
+        for h in range(NH):
+            qh, kh, vh, gh = (z[b, :, h * hd:(h + 1) * hd] for z in (q, k, v, go))
+            s = np.where(mask, np.float32(-1e9), qh @ kh.T / np.float32(np.sqrt(hd)))
+            e = np.exp((s - s.max(1, keepdims=True)).astype(np.float64)).astype(np.float32)
+            pr = e / e.sum(1, keepdims=True)
+            dp = gh @ vh.T
+            ds = np.where(mask, np.float32(0), pr * (dp - (pr * dp).sum(1, keepdims=True))) / np.float32(np.sqrt(hd))
+            left[h * hd:(h + 1) * hd] += (ds.T @ qh).sum(0)
+    assert q.dtype == ds.dtype == np.float32
+    a, r = np.linalg.norm(got[n1 + D * D:2 * n1]), np.linalg.norm(left / B)
+    log(f"  left over: {a:.3e}, numpy {r:.3e}")
+    assert a <= 1.5 * r
