@@ -1842,11 +1842,12 @@ __device__ __forceinline__ float exp32(float x) {
   return __builtin_ldexpf((float)p, (int)n);
 }
 
-template <int HD>
+template <int HD, bool SP = false>
 struct Fa {
   static constexpr int HX = HD / 16;              // 16-wide column groups
   static constexpr int P = HD + 4;                // LDS pitch: 16-byte aligned rows, conflict-free float4 reads
-  static constexpr int KS = HD <= 64 ? 64 : 32;   // rows per stage
+  // rows per stage: one 16-row tile per wave where the waves share them (SP)
+  static constexpr int KS = HD <= 64 || SP ? 64 : 32;
   static constexpr int RP = FA_NT / (HD / 4);     // rows per pass of the staging threads (a float4 each)
   static constexpr int NL = (KS + RP - 1) / RP;   // passes
 };
@@ -1861,41 +1862,43 @@ __device__ __forceinline__ float4 fa_load4(const float *__restrict__ p, int n) {
   return v;
 }
 
-// FULL: heads of exactly HD columns, 16-byte aligned.  Otherwise columns past
-// hd read as 0.  Rows past the end read as 0: their probabilities are 0, and 0
+// VEC: heads of a multiple of four columns, 16-byte aligned.  Columns past hd
+// read as 0, and so do rows past the end: their probabilities are 0, and 0
 // times an infinity of a re-read row would be NaN.
 
 // the lane's columns 16 x + 4*(l/16) .. +3 of row t
-template <int HD, bool FULL>
+template <int HD, bool VEC>
 __device__ __forceinline__ void fa_row(float4 (&v)[Fa<HD>::HX], const float *__restrict__ src, int t, int T, int D,
                                        int hd, int lane) {
   const int dl = 4 * (lane >> 4);
   const float *p = src + (int64_t)t * D + dl;
 #pragma unroll
   for (int x = 0; x < Fa<HD>::HX; ++x) {
-    if (FULL) v[x] = t < T ? *reinterpret_cast<const float4 *>(p + 16 * x) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (VEC)
+      v[x] = t < T && dl + 16 * x < hd ? *reinterpret_cast<const float4 *>(p + 16 * x) : make_float4(0.f, 0.f, 0.f, 0.f);
     else v[x] = fa_load4(p + 16 * x, t < T ? hd - dl - 16 * x : 0);
   }
 }
 
 // Staging of rows [k0, k0 + KS) of one matrix: thread t brings column group
 // t % (HD / 4) of rows t / (HD / 4) + q RP.
-template <int HD, bool FULL>
-__device__ __forceinline__ void fa_fetch(float4 (&v)[Fa<HD>::NL], const float *__restrict__ src, int k0, int T, int D,
-                                         int hd) {
-  using F = Fa<HD>;
+template <int HD, bool SP, bool VEC, int NL>
+__device__ __forceinline__ void fa_fetch(float4 (&v)[NL], const float *__restrict__ src, int k0, int T, int D, int hd) {
+  using F = Fa<HD, SP>;
+  static_assert(NL == F::NL, "staging passes");
   const int r = k0 + (int)threadIdx.x / (HD / 4), c = 4 * (threadIdx.x % (HD / 4));
 #pragma unroll
   for (int q = 0; q < F::NL; ++q) {
     const int t = r + q * F::RP;
     const float *p = src + (int64_t)t * D + c;
-    if (FULL) v[q] = t < T ? *reinterpret_cast<const float4 *>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (VEC) v[q] = t < T && c < hd ? *reinterpret_cast<const float4 *>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
     else v[q] = fa_load4(p, t < T ? hd - c : 0);
   }
 }
-template <int HD>
-__device__ __forceinline__ void fa_put(float *dst, const float4 (&v)[Fa<HD>::NL]) {
-  using F = Fa<HD>;
+template <int HD, bool SP, int NL>
+__device__ __forceinline__ void fa_put(float *dst, const float4 (&v)[NL]) {
+  using F = Fa<HD, SP>;
+  static_assert(NL == F::NL, "staging passes");
   const int r0 = threadIdx.x / (HD / 4), d = 4 * (threadIdx.x % (HD / 4));
   if (FA_NT % (HD / 4) && r0 >= F::RP) return;
 #pragma unroll
@@ -1937,7 +1940,7 @@ __device__ __forceinline__ void fa_zero(fx4 (&o)[Fa<HD>::HX]) {
   for (int x = 0; x < Fa<HD>::HX; ++x) o[x] = fx4{0.f, 0.f, 0.f, 0.f};
 }
 
-template <int HD, bool FULL>
+template <int HD, bool VEC>
 __device__ __forceinline__ void fa_store(float *__restrict__ G, const fx4 (&o)[Fa<HD>::HX], int64_t base, int t, int T,
                                          int D, int hd, int lane) {
   if (t >= T) return;
@@ -1945,8 +1948,8 @@ __device__ __forceinline__ void fa_store(float *__restrict__ G, const fx4 (&o)[F
 #pragma unroll
   for (int x = 0; x < Fa<HD>::HX; ++x) {
     const int d = 16 * x + 4 * (lane >> 4);
-    if (FULL) {
-      *reinterpret_cast<float4 *>(row + d) = make_float4(o[x][0], o[x][1], o[x][2], o[x][3]);
+    if (VEC) {
+      if (d < hd) *reinterpret_cast<float4 *>(row + d) = make_float4(o[x][0], o[x][1], o[x][2], o[x][3]);
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -1994,12 +1997,12 @@ __device__ __forceinline__ void fa_merge(fx4 (&o)[Fa<HD>::HX], float *buf) {
 // SP: the four waves share 16 rows and take every fourth 16-row tile of the
 // other side (their results meet in LDS), which gives a short batch four times
 // the workgroups; otherwise each wave has 16 rows of its own.
-template <int HD, bool SP, bool FULL>
+template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                        const float *__restrict__ V, float *__restrict__ O,
                                                        float2 *__restrict__ st, int T, int D, int NH, int hd,
                                                        int causal, int npair, int nb) {
-  using F = Fa<HD>;
+  using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
   __shared__ float wm[4][16], wl[4][16];
@@ -2010,21 +2013,21 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
   const int q0 = qb * RB + (SP ? 0 : 16 * w), qi = q0 + (lane & 15);
   const float is = 1.0f / (float)sqrt((double)hd);
   float4 qr[F::HX];
-  fa_row<HD, FULL>(qr, Q + base, qi, T, D, hd, lane);
+  fa_row<HD, VEC>(qr, Q + base, qi, T, D, hd, lane);
   fx4 o[F::HX];
   fa_zero<HD>(o);
   float m = -__builtin_inff(), l = 0.f;  // running maximum; the lane's own part of the sum
   const int kend = causal ? min(T, qb * RB + RB) : T;
   float4 kv[F::NL], vv[F::NL];
-  fa_fetch<HD, FULL>(kv, K + base, 0, T, D, hd);
-  fa_fetch<HD, FULL>(vv, V + base, 0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(kv, K + base, 0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(vv, V + base, 0, T, D, hd);
   for (int k0 = 0; k0 < kend; k0 += F::KS) {
-    fa_put<HD>(sk, kv);
-    fa_put<HD>(sv, vv);
+    fa_put<HD, SP>(sk, kv);
+    fa_put<HD, SP>(sv, vv);
     __syncthreads();
     if (k0 + F::KS < kend) {
-      fa_fetch<HD, FULL>(kv, K + base, k0 + F::KS, T, D, hd);
-      fa_fetch<HD, FULL>(vv, V + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(kv, K + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(vv, V + base, k0 + F::KS, T, D, hd);
     }
     const int jend = min(causal ? min(T, q0 + 16) : T, k0 + F::KS);  // the wave's live keys
     auto mine = [&](int kt) { return k0 + 16 * kt < jend && (!SP || (((k0 >> 4) + kt) & 3) == w); };
@@ -2089,7 +2092,7 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
   const float il = 1.0f / l;
 #pragma unroll
   for (int x = 0; x < F::HX; ++x) o[x] = o[x] * il;
-  fa_store<HD, FULL>(O, o, base, qi, T, D, hd, lane);
+  fa_store<HD, VEC>(O, o, base, qi, T, D, hd, lane);
   if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = make_float2(m, il);
 }
 
@@ -2123,13 +2126,13 @@ __device__ __forceinline__ float fa_rowdot(const float4 (&o)[Fa<HD>::HX], const 
 // then an exact zero, as in the reference.  A row of one stage of keys, where
 // few probabilities average that rounding, has the sum before its gQ and takes
 // it there too.
-template <int HD, bool SP, bool FULL>
+template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                          const float *__restrict__ V, const float *__restrict__ O,
                                                          const float *__restrict__ GO, float *__restrict__ GQ,
                                                          const float2 *__restrict__ st, float *__restrict__ dr, int T,
                                                          int D, int NH, int hd, int causal, int npair, int nb) {
-  using F = Fa<HD>;
+  using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
   __shared__ float sd[4][16];
@@ -2142,10 +2145,10 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
   float4 av[F::NL], bv[F::NL], za[F::HX], zb[F::HX];
   fx4 ga[F::HX];
   fa_zero<HD>(ga);
-  fa_row<HD, FULL>(za, O + base, ri, T, D, hd, lane);
-  fa_row<HD, FULL>(zb, GO + base, ri, T, D, hd, lane);
+  fa_row<HD, VEC>(za, O + base, ri, T, D, hd, lane);
+  fa_row<HD, VEC>(zb, GO + base, ri, T, D, hd, lane);
   const float c = fa_rowdot<HD>(za, zb, lane);
-  fa_row<HD, FULL>(za, Q + base, ri, T, D, hd, lane);
+  fa_row<HD, VEC>(za, Q + base, ri, T, D, hd, lane);
   const float2 ml = ri < T ? st[(int64_t)pair * T + ri] : make_float2(0.f, 0.f);
   const int kend = causal ? min(T, rb * RB + RB) : T;
   float dsum = 0.f;  // of P (dP - c)
@@ -2158,15 +2161,15 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
     return (sd[0][i] + sd[1][i]) + (sd[2][i] + sd[3][i]);
   };
   const bool one = kend <= F::KS;  // uniform over the workgroup
-  fa_fetch<HD, FULL>(av, K + base, 0, T, D, hd);
-  fa_fetch<HD, FULL>(bv, V + base, 0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(av, K + base, 0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(bv, V + base, 0, T, D, hd);
   for (int k0 = 0; k0 < kend; k0 += F::KS) {
-    fa_put<HD>(sa, av);
-    fa_put<HD>(sb, bv);
+    fa_put<HD, SP>(sa, av);
+    fa_put<HD, SP>(sb, bv);
     __syncthreads();
     if (k0 + F::KS < kend) {
-      fa_fetch<HD, FULL>(av, K + base, k0 + F::KS, T, D, hd);
-      fa_fetch<HD, FULL>(bv, V + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(av, K + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(bv, V + base, k0 + F::KS, T, D, hd);
     }
     if (r0 < T) {
       auto mine = [&](int kt) {  // uniform over the wave
@@ -2215,17 +2218,17 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
     if (w > 0) return;
   }
   if (lane < 16 && ri < T) dr[(int64_t)pair * T + ri] = c + dsum;
-  fa_store<HD, FULL>(GQ, ga, base, ri, T, D, hd, lane);
+  fa_store<HD, VEC>(GQ, ga, base, ri, T, D, hd, lane);
 }
 
 // Key blocks: gK and gV over the live queries, four products per tile pair.
-template <int HD, bool SP, bool FULL>
+template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                          const float *__restrict__ V, const float *__restrict__ GO,
                                                          float *__restrict__ GK, float *__restrict__ GV,
                                                          const float2 *__restrict__ st, const float *__restrict__ dr,
                                                          int T, int D, int NH, int hd, int causal, int npair, int nb) {
-  using F = Fa<HD>;
+  using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
   __shared__ __align__(16) float sm[F::KS], sl[F::KS], sd[F::KS];
@@ -2241,8 +2244,8 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
   fx4 ga[F::HX], gb[F::HX];
   fa_zero<HD>(ga);
   fa_zero<HD>(gb);
-  fa_row<HD, FULL>(za, K + base, ri, T, D, hd, lane);
-  fa_row<HD, FULL>(zb, V + base, ri, T, D, hd, lane);
+  fa_row<HD, VEC>(za, K + base, ri, T, D, hd, lane);
+  fa_row<HD, VEC>(zb, V + base, ri, T, D, hd, lane);
   const int i0 = causal ? rb * RB / F::KS * F::KS : 0;  // first stage with a live query
   // the saved statistics and d of a stage's queries: wave w its tile w
   float2 ml;
@@ -2253,12 +2256,12 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
     ml = t < T ? stp[t] : make_float2(0.f, 0.f);  // rows past the end: probability 0
     dq = t < T ? dp0[t] : 0.f;
   };
-  fa_fetch<HD, FULL>(av, Q + base, i0, T, D, hd);
-  fa_fetch<HD, FULL>(bv, GO + base, i0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(av, Q + base, i0, T, D, hd);
+  fa_fetch<HD, SP, VEC>(bv, GO + base, i0, T, D, hd);
   fetch_rows(i0);
   for (int k0 = i0; k0 < T; k0 += F::KS) {
-    fa_put<HD>(sa, av);
-    fa_put<HD>(sb, bv);
+    fa_put<HD, SP>(sa, av);
+    fa_put<HD, SP>(sb, bv);
     if (w < KT && lane < 16) {
       sm[16 * w + lane] = ml.x;
       sl[16 * w + lane] = ml.y;
@@ -2266,8 +2269,8 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
     }
     __syncthreads();
     if (k0 + F::KS < T) {
-      fa_fetch<HD, FULL>(av, Q + base, k0 + F::KS, T, D, hd);
-      fa_fetch<HD, FULL>(bv, GO + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(av, Q + base, k0 + F::KS, T, D, hd);
+      fa_fetch<HD, SP, VEC>(bv, GO + base, k0 + F::KS, T, D, hd);
       fetch_rows(k0 + F::KS);
     }
     if (r0 < T) {
@@ -2315,8 +2318,8 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
     fa_merge<HD>(gb, sh);
     if (w > 0) return;
   }
-  fa_store<HD, FULL>(GK, ga, base, ri, T, D, hd, lane);
-  fa_store<HD, FULL>(GV, gb, base, ri, T, D, hd, lane);
+  fa_store<HD, VEC>(GK, ga, base, ri, T, D, hd, lane);
+  fa_store<HD, VEC>(GV, gb, base, ri, T, D, hd, lane);
 }
 
 static bool fa_supported(int D, int NH) { return NH > 0 && D % NH == 0 && D / NH <= 128; }
@@ -2326,7 +2329,7 @@ size_t attn_work_floats(int B, int T, int D, int NH) {
   return fa_supported(D, NH) ? 3 * rows : 2 * rows * T;  // (maximum, 1 / sum) and d; scores and their gradients
 }
 
-template <int HD, bool SP, bool FULL>
+template <int HD, bool SP, bool VEC>
 static hipError_t fa_launch(const float *Q, const float *K, const float *V, float *O, const float *GO, float *GQ,
                             float *GK, float *GV, float *S, int B, int T, int D, int NH, int causal, hipStream_t s) {
   const int hd = D / NH, rb = SP ? 16 : FA_B, nb = (T + rb - 1) / rb;
@@ -2336,15 +2339,15 @@ static hipError_t fa_launch(const float *Q, const float *K, const float *V, floa
   float *dr = S + 2 * np * T;
   const dim3 grid((unsigned)(np * nb)), block(FA_NT);
   if (!GO) {
-    hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, O, st, T, D, NH, hd, causal, (int)np,
+    hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, O, st, T, D, NH, hd, causal, (int)np,
                        nb);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((fa_bwd_q_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, O, GO, GQ, st, dr, T, D, NH, hd,
+  hipLaunchKernelGGL((fa_bwd_q_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, O, GO, GQ, st, dr, T, D, NH, hd,
                      causal, (int)np, nb);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((fa_bwd_k_kernel<HD, SP, FULL>), grid, block, 0, s, Q, K, V, GO, GK, GV, st, dr, T, D, NH, hd,
+  hipLaunchKernelGGL((fa_bwd_k_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, GO, GK, GV, st, dr, T, D, NH, hd,
                      causal, (int)np, nb);
   return hipGetLastError();
 }
@@ -2354,25 +2357,27 @@ static hipError_t fa_launch(const float *Q, const float *K, const float *V, floa
 static hipError_t fa_run(const float *Q, const float *K, const float *V, float *O, const float *GO, float *GQ,
                          float *GK, float *GV, float *S, int B, int T, int D, int NH, int causal, hipStream_t s) {
   const int hd = D / NH;
-  // up to 512 workgroups of 64 rows leave SIMDs with one wave or none: 16-row
-  // workgroups then (B 1, T 1024, one 64-wide head 229 -> 127 us; B 4, T 512,
-  // 8 heads 232 -> 216), not beyond (768 workgroups, B 2, T 1000, 12 heads:
-  // 293 -> 325), nor with 32-row stages, where half the waves would idle (80
-  // columns 160 -> 171), nor where the other side is a tile or two
-  const bool sp = T > 32 && (int64_t)B * NH * ((T + FA_B - 1) / FA_B) * (GO ? 2 : 1) <= 512;
+  // Up to 512 workgroups of 64 rows (256 of the backward, whose waves hold more)
+  // leave SIMDs with one wave or none: 16-row workgroups then (B 1, T 1024, one
+  // 64-wide head 229 -> 127 us; B 4, T 512, 8 heads 232 -> 216), not beyond
+  // (forward, 768 workgroups, B 2, T 1000, 12 heads: 293 -> 325; backward, 512
+  // workgroups, B 2, T 2000, 8 heads: 1162 -> 1377), nor where the other side is
+  // a tile or two.  Heads beyond 64, whose larger stages take most of a CU's LDS
+  // or registers, only where 64-row workgroups leave CUs empty (B 1, T 1024, 8
+  // heads of 128 670 -> 408; at 256 workgroups, B 8, T 256, 480 -> 570).
+  const int64_t wg = (int64_t)B * NH * ((T + FA_B - 1) / FA_B);
+  const bool sp = T > 32 && (hd > 64 ? wg < 256 : wg <= (GO ? 256 : 512));
   uintptr_t al = reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
                  reinterpret_cast<uintptr_t>(O);
   if (GO)
     al |= reinterpret_cast<uintptr_t>(GO) | reinterpret_cast<uintptr_t>(GQ) | reinterpret_cast<uintptr_t>(GK) |
           reinterpret_cast<uintptr_t>(GV);
-  const bool a16 = (al & 15) == 0;
+  const bool vec = (al & 15) == 0 && hd % 4 == 0;
 #define FA_CASE(H)                                                                                        \
   if (hd <= H) {                                                                                          \
-    if (hd == H && a16)                                                                                   \
-      return sp && H <= 64                                                                                \
-                 ? fa_launch<H, (H <= 64), true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s)   \
-                 : fa_launch<H, false, true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);      \
-    return fa_launch<H, false, false>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);             \
+    if (!vec) return fa_launch<H, false, false>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);   \
+    return sp ? fa_launch<H, true, true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s)           \
+              : fa_launch<H, false, true>(Q, K, V, O, GO, GQ, GK, GV, S, B, T, D, NH, causal, s);         \
   }
   FA_CASE(32);
   FA_CASE(48);

@@ -61,6 +61,16 @@ def test_attn_sizes(dev, oracle, B, T, D, NH, causal):
         assert max_rel(got[i * n1:i * n1 + D * D], ref[:D * D]) <= TOL, name
 
 
+# heads of a multiple of four columns below the padded width (16-byte accesses),
+# heads beyond 64 with 16-row workgroups (fewer than 256 of 64 rows) and 64-row ones
+@pytest.mark.parametrize("B,T,D,NH,causal", [
+    (1, 97, 24, 1, 1), (2, 70, 80, 2, 0), (1, 130, 100, 1, 0), (2, 65, 120, 1, 1), (130, 65, 48, 2, 1),
+    (1, 193, 128, 1, 1), (1, 129, 80, 1, 0), (2, 64, 192, 2, 1), (1, 49, 68, 1, 0), (64, 66, 256, 2, 1),
+    (64, 65, 168, 2, 0), (130, 40, 96, 1, 1), (1, 131, 4, 1, 1)])
+def test_attn_head_widths(dev, oracle, B, T, D, NH, causal):
+    test_attn_sizes(dev, oracle, B, T, D, NH, causal)
+
+
 def test_attn_single_key_rows_have_no_score_gradient(dev):
     """Under the causal mask token 0 attends to itself alone: its probability is
     1 and gradScore an exact zero, so with a gradient on token 0 only the query
