@@ -1804,9 +1804,7 @@ bool attn_supported(int T, int D, int NH) {
 // ---------------------------------------------------------------------------
 // Attention of any sequence length with heads of up to 128 (what the kernels
 // above do not hold in LDS at once), on fp32 MFMA 16x16x4 with their operand
-// layouts and the same mask convention (key tiles that lie wholly above the
-// diagonal contribute exact zeros).  Nothing of size T x T is written: the
-// forward keeps a running row maximum and sum over stages of keys and leaves
+// layouts.  Nothing of size T x T is written: the forward keeps a running row maximum and sum over stages of keys and leaves
 // (maximum, 1 / sum) per row for the backward, which recomputes the
 // probabilities.  A workgroup is four waves that share the staged rows of the
 // other side in LDS.
@@ -1820,6 +1818,13 @@ bool attn_supported(int T, int D, int NH) {
 // ---------------------------------------------------------------------------
 constexpr int FA_B = 64;    // rows per workgroup (16 per wave) where they fill the chip
 constexpr int FA_NT = 256;
+// A masked key scores -1e9: its weight is an exact zero unless the row's maximum
+// is about that low itself.  A workgroup with such a row (or one without a
+// finite sum) takes the tiles above the diagonal too.
+constexpr float FA_MASKED = -0.99e9f;
+__device__ __forceinline__ bool fa_whole(const float2 &ml) {  // (maximum, 1 / sum) of an ordinary row
+  return ml.x > FA_MASKED && ml.y < __builtin_inff();
+}
 
 // float32(exp(x)) for x <= 0 in float64 after Cody and Waite's reduction x = n
 // ln 2 + r: the Taylor polynomial of degree 9 in |r| <= ln 2 / 2 is within
@@ -2075,6 +2080,36 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
     }
     __syncthreads();
   }
+  if (causal) {  // rows that give masked keys weight: those of the tiles above the diagonal too
+    float mr = m;
+    if (SP) {
+      if (lane < 16) wm[w][lane] = m;
+      __syncthreads();
+      const int i = lane & 15;
+      mr = fmaxf(fmaxf(wm[0][i], wm[1][i]), fmaxf(wm[2][i], wm[3][i]));
+    }
+    if (__syncthreads_or(qi < T && !(mr > FA_MASKED))) {
+      for (int k0 = qb * RB / F::KS * F::KS; k0 < T; k0 += F::KS) {
+        fa_fetch<HD, SP, VEC>(vv, V + base, k0, T, D, hd);
+        __syncthreads();
+        fa_put<HD, SP>(sv, vv);
+        __syncthreads();
+        for (int kt = 0; kt < F::KS / 16; ++kt) {
+          const int jb = k0 + 16 * kt;
+          if (q0 >= T || jb < q0 + 16 || jb >= T || (SP && ((jb >> 4) & 3) != w)) continue;  // uniform over the wave
+          const float mn = fmaxf(m, -1e9f), al = exp32(m - mn), p = exp32(-1e9f - mn);
+          fx4 e;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) e[r] = jb + 4 * (lane >> 4) + r < T ? p : 0.f;
+          l = __builtin_fmaf(l, al, (e[0] + e[1]) + (e[2] + e[3]));
+#pragma unroll
+          for (int x = 0; x < F::HX; ++x) o[x] = o[x] * al;
+          fa_acc<HD>(o, sv, e, kt, lane);
+          m = mn;
+        }
+      }
+    }
+  }
   l = fa_sum4(l);
   if (SP) {  // the waves' parts on a common maximum
     if (lane < 16) wm[w][lane] = m;
@@ -2130,8 +2165,9 @@ template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                          const float *__restrict__ V, const float *__restrict__ O,
                                                          const float *__restrict__ GO, float *__restrict__ GQ,
-                                                         const float2 *__restrict__ st, float *__restrict__ dr, int T,
-                                                         int D, int NH, int hd, int causal, int npair, int nb) {
+                                                         const float2 *__restrict__ st, float *__restrict__ dr,
+                                                         float *__restrict__ fl, int T, int D, int NH, int hd,
+                                                         int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
@@ -2147,7 +2183,7 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
   fa_zero<HD>(ga);
   fa_row<HD, VEC>(za, O + base, ri, T, D, hd, lane);
   fa_row<HD, VEC>(zb, GO + base, ri, T, D, hd, lane);
-  const float c = fa_rowdot<HD>(za, zb, lane);
+  float c = fa_rowdot<HD>(za, zb, lane);
   fa_row<HD, VEC>(za, Q + base, ri, T, D, hd, lane);
   const float2 ml = ri < T ? st[(int64_t)pair * T + ri] : make_float2(0.f, 0.f);
   const int kend = causal ? min(T, rb * RB + RB) : T;
@@ -2160,64 +2196,78 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
     const int i = lane & 15;
     return (sd[0][i] + sd[1][i]) + (sd[2][i] + sd[3][i]);
   };
-  const bool one = kend <= F::KS;  // uniform over the workgroup
-  fa_fetch<HD, SP, VEC>(av, K + base, 0, T, D, hd);
-  fa_fetch<HD, SP, VEC>(bv, V + base, 0, T, D, hd);
-  for (int k0 = 0; k0 < kend; k0 += F::KS) {
-    fa_put<HD, SP>(sa, av);
-    fa_put<HD, SP>(sb, bv);
-    __syncthreads();
-    if (k0 + F::KS < kend) {
-      fa_fetch<HD, SP, VEC>(av, K + base, k0 + F::KS, T, D, hd);
-      fa_fetch<HD, SP, VEC>(bv, V + base, k0 + F::KS, T, D, hd);
-    }
-    if (r0 < T) {
-      auto mine = [&](int kt) {  // uniform over the wave
-        const int jb = k0 + 16 * kt;
-        return jb < T && !(causal && jb > r0 + 15) && (!SP || ((jb >> 4) & 3) == w);
-      };
-      fx4 ps[KT], ds[KT];
+  // gO . o holds the masked keys' weights, which d does not: where a row has any,
+  // d is summed in a pass of its own
+  const bool masked = causal && __syncthreads_or(ri < T && !fa_whole(ml));
+  if (causal && threadIdx.x == 0) fl[(int64_t)pair * nb + rb] = masked ? 1.f : 0.f;
+  const bool one = kend <= F::KS && !masked;  // uniform over the workgroup
+  for (int ph = masked ? 0 : 1; ph < 2; ++ph) {
+    if (ph == 0) c = 0.f;
+    fa_fetch<HD, SP, VEC>(av, K + base, 0, T, D, hd);
+    fa_fetch<HD, SP, VEC>(bv, V + base, 0, T, D, hd);
+    for (int k0 = 0; k0 < kend; k0 += F::KS) {
+      fa_put<HD, SP>(sa, av);
+      fa_put<HD, SP>(sb, bv);
+      __syncthreads();
+      if (k0 + F::KS < kend) {
+        fa_fetch<HD, SP, VEC>(av, K + base, k0 + F::KS, T, D, hd);
+        fa_fetch<HD, SP, VEC>(bv, V + base, k0 + F::KS, T, D, hd);
+      }
+      if (r0 < T) {
+        auto mine = [&](int kt) {  // uniform over the wave
+          const int jb = k0 + 16 * kt;
+          return jb < T && !(causal && jb > r0 + 15) && (!SP || ((jb >> 4) & 3) == w);
+        };
+        fx4 ps[KT], ds[KT];
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        if (!mine(kt)) continue;
-        const int jb = k0 + 16 * kt;
-        const fx4 s = fa_tile<HD>(sa, za, kt, lane), dp = fa_tile<HD>(sb, zb, kt, lane);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ps[kt][r] = exp32(s[r] * is - ml.x) * ml.y;
-          ds[kt][r] = ps[kt][r] * (dp[r] - c);
-        }
-        if (jb + 15 >= T || r0 + 15 >= T || (causal && jb + 15 > r0)) {  // uniform: a tile at an edge
+        for (int kt = 0; kt < KT; ++kt) {
+          if (!mine(kt)) continue;
+          const int jb = k0 + 16 * kt;
+          const fx4 s = fa_tile<HD>(sa, za, kt, lane), dp = fa_tile<HD>(sb, zb, kt, lane);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int j = jb + dl + r;
-            const bool live = j < T && ri < T && !(causal && j > ri);
-            ps[kt][r] = live ? ps[kt][r] : 0.f;
-            ds[kt][r] = live ? ds[kt][r] : 0.f;
+            ps[kt][r] = exp32(s[r] * is - ml.x) * ml.y;
+            ds[kt][r] = ps[kt][r] * (dp[r] - c);
           }
+          if (jb + 15 >= T || r0 + 15 >= T || (causal && jb + 15 > r0)) {  // uniform: a tile at an edge
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int j = jb + dl + r;
+              const bool live = j < T && ri < T && !(causal && j > ri);
+              ps[kt][r] = live ? ps[kt][r] : 0.f;
+              ds[kt][r] = live ? ds[kt][r] : 0.f;
+            }
+          }
+          dsum += (ds[kt][0] + ds[kt][1]) + (ds[kt][2] + ds[kt][3]);
         }
-        dsum += (ds[kt][0] + ds[kt][1]) + (ds[kt][2] + ds[kt][3]);
-      }
-      if (one) dsum = row_sum(dsum);
-      fx4 gs[F::HX];  // the stage's own sums
-      fa_zero<HD>(gs);
+        if (one) dsum = row_sum(dsum);
+        if (ph) {
+          fx4 gs[F::HX];  // the stage's own sums
+          fa_zero<HD>(gs);
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        if (!mine(kt)) continue;
-        if (one) ds[kt] = ds[kt] - ps[kt] * dsum;
-        fa_acc<HD>(gs, sa, ds[kt] * is, kt, lane);  // gQ_i += gradScore_ij k_j
-      }
+          for (int kt = 0; kt < KT; ++kt) {
+            if (!mine(kt)) continue;
+            if (one) ds[kt] = ds[kt] - ps[kt] * dsum;
+            fa_acc<HD>(gs, sa, ds[kt] * is, kt, lane);  // gQ_i += gradScore_ij k_j
+          }
 #pragma unroll
-      for (int x = 0; x < F::HX; ++x) ga[x] = ga[x] + gs[x];
+          for (int x = 0; x < F::HX; ++x) ga[x] = ga[x] + gs[x];
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
+    if (ph == 0) {
+      c = row_sum(dsum);
+      dsum = 0.f;
+      __syncthreads();
+    }
   }
-  if (!one) dsum = row_sum(dsum);
+  if (!one && !masked) dsum = row_sum(dsum);
   if (SP) {
     fa_merge<HD>(ga, sh);
     if (w > 0) return;
   }
-  if (lane < 16 && ri < T) dr[(int64_t)pair * T + ri] = c + dsum;
+  if (lane < 16 && ri < T) dr[(int64_t)pair * T + ri] = masked ? c : c + dsum;
   fa_store<HD, VEC>(GQ, ga, base, ri, T, D, hd, lane);
 }
 
@@ -2227,7 +2277,8 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
                                                          const float *__restrict__ V, const float *__restrict__ GO,
                                                          float *__restrict__ GK, float *__restrict__ GV,
                                                          const float2 *__restrict__ st, const float *__restrict__ dr,
-                                                         int T, int D, int NH, int hd, int causal, int npair, int nb) {
+                                                         const float *__restrict__ fl, int T, int D, int NH, int hd,
+                                                         int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
@@ -2246,7 +2297,14 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
   fa_zero<HD>(gb);
   fa_row<HD, VEC>(za, K + base, ri, T, D, hd, lane);
   fa_row<HD, VEC>(zb, V + base, ri, T, D, hd, lane);
-  const int i0 = causal ? rb * RB / F::KS * F::KS : 0;  // first stage with a live query
+  // earlier queries give these keys no weight unless a query block says so
+  bool all = !causal;
+  if (causal) {
+    bool any = false;
+    for (int i = threadIdx.x; i <= rb; i += FA_NT) any = any || fl[(int64_t)pair * nb + i] != 0.f;
+    all = __syncthreads_or(any);
+  }
+  const int i0 = all ? 0 : rb * RB / F::KS * F::KS;  // first stage with a live query
   // the saved statistics and d of a stage's queries: wave w its tile w
   float2 ml;
   float dq;
@@ -2280,26 +2338,32 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
 #pragma unroll
       for (int qt = 0; qt < KT; ++qt) {
         const int ib = k0 + 16 * qt;
-        if (ib >= T || (causal && ib + 15 < r0) || (SP && ((ib >> 4) & 3) != w)) continue;  // uniform over the wave
+        if (ib >= T || (!all && ib + 15 < r0) || (SP && ((ib >> 4) & 3) != w)) continue;  // uniform over the wave
         fx4 s = fa_tile<HD>(sa, za, qt, lane), dp = fa_tile<HD>(sb, zb, qt, lane);
         const float4 m4 = *reinterpret_cast<const float4 *>(sm + 16 * qt + dl);
         const float4 l4 = *reinterpret_cast<const float4 *>(sl + 16 * qt + dl);
         const float4 d4 = *reinterpret_cast<const float4 *>(sd + 16 * qt + dl);
         const float mm[4] = {m4.x, m4.y, m4.z, m4.w}, ll[4] = {l4.x, l4.y, l4.z, l4.w};
         const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+        const bool edge = ib + 15 >= T || r0 + 15 >= T || (causal && r0 + 15 > ib);  // uniform
+        s = s * is;
+        if (causal && r0 + 15 > ib) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[r] = ri > ib + dl + r ? -1e9f : s[r];
+        }
         fx4 ds;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[r] = exp32(s[r] * is - mm[r]) * ll[r];
+          s[r] = exp32(s[r] - mm[r]) * ll[r];
           ds[r] = s[r] * (dp[r] - dd[r]) * is;
         }
-        if (ib + 15 >= T || r0 + 15 >= T || (causal && r0 + 15 > ib)) {  // uniform: a tile at an edge
+        if (edge) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int i = ib + dl + r;
-            const bool live = i < T && ri < T && !(causal && ri > i);
-            s[r] = live ? s[r] : 0.f;
-            ds[r] = live ? ds[r] : 0.f;
+            const bool in = i < T && ri < T;
+            s[r] = in ? s[r] : 0.f;
+            ds[r] = in && !(causal && ri > i) ? ds[r] : 0.f;
           }
         }
         fa_acc<HD>(gbs, sb, s, qt, lane);   // gV_j += p_ij gO_i
@@ -2326,7 +2390,8 @@ static bool fa_supported(int D, int NH) { return NH > 0 && D % NH == 0 && D / NH
 
 size_t attn_work_floats(int B, int T, int D, int NH) {
   const size_t rows = (size_t)B * NH * T;
-  return fa_supported(D, NH) ? 3 * rows : 2 * rows * T;  // (maximum, 1 / sum) and d; scores and their gradients
+  // (maximum, 1 / sum), d and a flag per block of at least 16 rows; or scores and their gradients
+  return fa_supported(D, NH) ? 3 * rows + (size_t)B * NH * ((T + 15) / 16) : 2 * rows * T;
 }
 
 template <int HD, bool SP, bool VEC>
@@ -2336,19 +2401,19 @@ static hipError_t fa_launch(const float *Q, const float *K, const float *V, floa
   const int64_t np = (int64_t)B * NH;
   if (np * nb * 2 > 0x7fffffff) return hipErrorInvalidValue;
   float2 *st = reinterpret_cast<float2 *>(S);
-  float *dr = S + 2 * np * T;
+  float *dr = S + 2 * np * T, *fl = S + 3 * np * T;
   const dim3 grid((unsigned)(np * nb)), block(FA_NT);
   if (!GO) {
     hipLaunchKernelGGL((fa_fwd_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, O, st, T, D, NH, hd, causal, (int)np,
                        nb);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((fa_bwd_q_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, O, GO, GQ, st, dr, T, D, NH, hd,
-                     causal, (int)np, nb);
+  hipLaunchKernelGGL((fa_bwd_q_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, O, GO, GQ, st, dr, fl, T, D, NH,
+                     hd, causal, (int)np, nb);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((fa_bwd_k_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, GO, GK, GV, st, dr, T, D, NH, hd,
-                     causal, (int)np, nb);
+  hipLaunchKernelGGL((fa_bwd_k_kernel<HD, SP, VEC>), grid, block, 0, s, Q, K, V, GO, GK, GV, st, dr, fl, T, D, NH,
+                     hd, causal, (int)np, nb);
   return hipGetLastError();
 }
 

@@ -138,3 +138,45 @@ def test_attn_vanishing_sums(dev, T, D, NH, causal):
     a, r = np.linalg.norm(got[n1 + D * D:2 * n1]), np.linalg.norm(left / B)
     log(f"  left over: {a:.3e}, numpy {r:.3e}")
     assert a <= 1.5 * r
+
+
+@pytest.mark.parametrize("T,D,NH", [(150, 64, 2), (70, 96, 1), (200, 24, 1), (40, 128, 1), (530, 16, 1)])
+@pytest.mark.parametrize("rows", [1, 300])
+def test_attn_masked_keys_with_weight(dev, oracle, T, D, NH, rows):
+    """A masked key scores -1e9, which weighs nothing beside ordinary scores.
+    Rows whose own keys all score lower (here by q_0 = 1e6, k_0 = -1e6 in each
+    head) divide their weight among the masked keys, in every tile, and their
+    value gradient too.  Column 0 of each head's query gradient is left out, and
+    with it the input gradient of the column that sets it: rounding times 1e6."""
+    B, hd = 150 if rows > 1 else 1, D // NH  # few and many workgroups
+    log(f"attention masked weights T={T} D={D} heads={NH} B={B}")
+    rng = np.random.default_rng(T + D)
+    n1 = D * D + D
+    w = [rng.normal(size=n1).astype(np.float32) / np.float32(np.sqrt(D)) for _ in range(4)]
+    for i in range(2):
+        W, b = w[i][:D * D].reshape(D, D), w[i][D * D:]
+        W[:, 0] = 0
+        W[::hd] = 0
+        b[::hd] = 0 if i == 0 else -1e6
+        if i == 0:
+            W[::hd, 0] = 1e6
+    p = np.concatenate(w)
+    x, g = (rng.normal(size=(1, T, D)).astype(np.float32) for _ in range(2))
+    x[:, :, 0] = 0
+    x[:, [0, 3, T // 2, T - 2], 0] = 1
+    net = oracle.Net([oracle.spec(oracle.LAYER_MHA, dim=D, num_heads=NH, seq_len=T, causal=1, use_rope=0)],
+                     oracle.LOSS_MSE)
+    net.params[:] = p
+    out_r, gin_r = net.accumulate_grad(x.reshape(1, -1), g.reshape(1, -1), 1, T * D, T * D)
+    gr = net.grads.copy()
+    out, got, gin = _mha(dev, B, T, D, NH, 1, p, np.tile(x.reshape(1, -1), (B, 1)), np.tile(g.reshape(1, -1), (B, 1)))
+    keep = np.ones(D, bool)
+    keep[0] = False
+    for r in (0, B - 1):
+        assert max_rel(out[r], out_r[0]) <= TOL
+        assert max_rel(gin[r].reshape(T, D)[:, keep], gin_r.reshape(T, D)[:, keep]) <= TOL
+    rows_ = np.arange(D) % hd != 0
+    for i, name in ((0, "wQ"), (2, "wV"), (3, "wOut")):
+        a, b = (z[i * n1:i * n1 + D * D].reshape(D, D) for z in (got, gr))
+        k = rows_ if i == 0 else slice(None)
+        assert max_rel(a[k], b[k]) <= TOL, name
