@@ -59,18 +59,24 @@ __device__ __forceinline__ void gru_fma4(float4 &s, const float4 &w, float x) {
   s.w = __builtin_fmaf(w.w, x, s.w);
 }
 
-// row k, columns 4c .. 4c+3 of W (pitch ld, columns below H); zero past the
-// matrix.  v4: H % 4 == 0 and W 16-byte aligned.
-__device__ __forceinline__ float4 gru_w4(const float *__restrict__ W, int ld, int k, int K, int c, int H,
-                                         bool v4) {
+// 16-byte load from any float's address (global_load_dwordx4 asks for 4 bytes)
+typedef float gru_fx4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 gru_ld4(const float *p) {
+  const gru_fx4 v = *reinterpret_cast<const gru_fx4 *>(p);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// row k, columns 4c .. 4c+3 of W (K rows, pitch ld, columns below H, 4c < H);
+// zero past the last row.  Columns past H come from what follows in memory
+// (their sums are never read), but not past the last row's end.
+__device__ __forceinline__ float4 gru_w4(const float *__restrict__ W, int ld, int k, int K, int c, int H) {
   float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
   if (k >= K) return w;
   const float *p = W + (size_t)k * ld + 4 * c;
-  if (v4) return 4 * c < H ? *reinterpret_cast<const float4 *>(p) : w;
-  if (4 * c < H) w.x = p[0];
+  if (4 * c + 3 < H || k + 1 < K) return gru_ld4(p);
+  w.x = p[0];
   if (4 * c + 1 < H) w.y = p[1];
   if (4 * c + 2 < H) w.z = p[2];
-  if (4 * c + 3 < H) w.w = p[3];
   return w;
 }
 
@@ -83,23 +89,23 @@ __device__ __forceinline__ void gru_rows4(float4 &s, const float4 *w, const floa
 }
 
 // s += sum over rows e in [e0, rows) of the share, read from global memory,
-// eight 16-byte loads in flight (W holds K rows; H % 4 == 0 and W 16-byte
-// aligned with v4)
+// eight 16-byte loads in flight (W holds K rows).  A scalar form for widths
+// that are no multiple of 4 had one row in flight: H 513, T 30, B 64 8085 us,
+// with unaligned loads 1480 (H 512: 1158).
 __device__ __forceinline__ void gru_stream(float4 &s, const float *__restrict__ W, int ld, int k0, int e0,
-                                           int rows, int K, int c, int H, bool v4, const float *v) {
-  const int e1 = min(rows, K - k0);  // rows of the matrix
+                                           int rows, int K, int c, int H, const float *v) {
+  const int e1 = min(rows, K - k0);                                  // rows of the matrix
+  const int ev = e1 - (4 * c + 3 >= H && k0 + e1 == K ? 1 : 0);      // of them those read whole
   int e = e0;
-  if (v4) {
-    const float *p = W + (size_t)(k0 + e0) * ld + 4 * c;
-    for (; e + 8 <= e1; e += 8, p += 8 * (size_t)ld) {
-      float4 w[8];
+  const float *p = W + (size_t)(k0 + e0) * ld + 4 * c;
+  for (; e + 8 <= ev; e += 8, p += 8 * (size_t)ld) {
+    float4 w[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = *reinterpret_cast<const float4 *>(p + u * (size_t)ld);
-      gru_rows4(s, w, *reinterpret_cast<const float4 *>(v + k0 + e));
-      gru_rows4(s, w + 4, *reinterpret_cast<const float4 *>(v + k0 + e + 4));
-    }
+    for (int u = 0; u < 8; ++u) w[u] = gru_ld4(p + u * (size_t)ld);
+    gru_rows4(s, w, *reinterpret_cast<const float4 *>(v + k0 + e));
+    gru_rows4(s, w + 4, *reinterpret_cast<const float4 *>(v + k0 + e + 4));
   }
-  for (; e < e1; ++e) gru_fma4(s, gru_w4(W, ld, k0 + e, K, c, H, v4), v[k0 + e]);
+  for (; e < e1; ++e) gru_fma4(s, gru_w4(W, ld, k0 + e, K, c, H), v[k0 + e]);
 }
 
 // xw [B*T][3H] = b + Wx x_t (from the GEMM); WhT [H][2H]; writes act [B*T][3H]
@@ -121,17 +127,16 @@ void gru_fwd_kernel(const float *__restrict__ xw, const float *__restrict__ WhT,
   float4 *Wl = reinterpret_cast<float4 *>(part + NQ * 2 * HC);      // [lrows][GB * NQ]
   const int c = tid % GB, q = tid / GB, k0 = q * rows, np = GB * NQ;
   const bool mv = tid < np;
-  const bool v4 = (H & 3) == 0;  // WhT is the caller's 16-byte aligned scratch
   float4 wr[RR], wu[RU];
 #pragma unroll
   for (int e = 0; e < RR; ++e)
-    wr[e] = mv && e < rows ? gru_w4(WhT + H, 2 * H, k0 + e, H, c, H, v4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    wr[e] = mv && e < rows ? gru_w4(WhT + H, 2 * H, k0 + e, H, c, H) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int e = 0; e < RU; ++e)
-    wu[e] = mv && e < rows ? gru_w4(WhT, 2 * H, k0 + e, H, c, H, v4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    wu[e] = mv && e < rows ? gru_w4(WhT, 2 * H, k0 + e, H, c, H) : make_float4(0.f, 0.f, 0.f, 0.f);
   if (mv)
     for (int e = 0; e < pl.lrows; ++e)
-      Wl[e * np + tid] = gru_w4(WhT, 2 * H, k0 + RU + e, H, c, H, v4);
+      Wl[e * np + tid] = gru_w4(WhT, 2 * H, k0 + RU + e, H, c, H);
   for (int i = tid; i < HP; i += nt) hs[i] = srh[i] = 0.0f;  // GRU.Reset (gru.go:171-180); the pad stays 0
   const float *xb = xw + (size_t)b * T * 3 * H;
   for (int i = tid; i < 3 * H; i += nt) xs[i] = xb[i];
@@ -171,8 +176,8 @@ void gru_fwd_kernel(const float *__restrict__ xw, const float *__restrict__ WhT,
         }
       }
       if (BIG) {
-        gru_stream(su, WhT, 2 * H, k0, RU + pl.lrows, rows, H, c, H, v4, hs);
-        gru_stream(sr, WhT + H, 2 * H, k0, RR, rows, H, c, H, v4, hs);
+        gru_stream(su, WhT, 2 * H, k0, RU + pl.lrows, rows, H, c, H, hs);
+        gru_stream(sr, WhT + H, 2 * H, k0, RR, rows, H, c, H, hs);
       }
       *reinterpret_cast<float4 *>(part + q * 2 * HC + 4 * c) = su;
       *reinterpret_cast<float4 *>(part + q * 2 * HC + HC + 4 * c) = sr;
@@ -201,7 +206,7 @@ void gru_fwd_kernel(const float *__restrict__ xw, const float *__restrict__ WhT,
 #pragma unroll
       for (int e = 0; e < RR; e += 4)
         if (e < rows) gru_rows4(sc, wr + e, *reinterpret_cast<const float4 *>(srh + k0 + e));
-      if (BIG) gru_stream(sc, WhT + H, 2 * H, k0, RR, rows, H, c, H, v4, srh);
+      if (BIG) gru_stream(sc, WhT + H, 2 * H, k0, RR, rows, H, c, H, srh);
       *reinterpret_cast<float4 *>(part + q * 2 * HC + 4 * c) = sc;
     }
     lds_barrier();
@@ -232,7 +237,7 @@ void gru_fwd_kernel(const float *__restrict__ xw, const float *__restrict__ WhT,
 template <int RW, bool BIG>
 __global__ __launch_bounds__(GR_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gru_bwd_kernel(const float *__restrict__ g, const float *__restrict__ act, const float *__restrict__ hprev,
-                    const float *__restrict__ Wh, float *__restrict__ dG, int T, int H, int seq, int v4a,
+                    const float *__restrict__ Wh, float *__restrict__ dG, int T, int H, int seq,
                     GruPlan pl) {
   extern __shared__ __align__(16) float gsm[];
   const int GB = pl.GB, NQ = pl.NQ, rows = pl.rows, HC = 4 * GB, VP = NQ * rows;
@@ -241,13 +246,13 @@ void gru_bwd_kernel(const float *__restrict__ g, const float *__restrict__ act, 
   float *part = vs + VP;           // [NQ][HC]
   float4 *Wl = reinterpret_cast<float4 *>(part + NQ * HC);
   const int c = tid % GB, q = tid / GB, k0 = q * rows, np = GB * NQ;
-  const bool mv = tid < np, v4 = v4a != 0;
+  const bool mv = tid < np;
   float4 w[RW];
 #pragma unroll
   for (int e = 0; e < RW; ++e)
-    w[e] = mv && e < rows ? gru_w4(Wh, H, k0 + e, 2 * H, c, H, v4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    w[e] = mv && e < rows ? gru_w4(Wh, H, k0 + e, 2 * H, c, H) : make_float4(0.f, 0.f, 0.f, 0.f);
   if (mv)
-    for (int e = 0; e < pl.lrows; ++e) Wl[e * np + tid] = gru_w4(Wh, H, k0 + RW + e, 2 * H, c, H, v4);
+    for (int e = 0; e < pl.lrows; ++e) Wl[e * np + tid] = gru_w4(Wh, H, k0 + RW + e, 2 * H, c, H);
   for (int i = tid; i < VP; i += nt) vs[i] = 0.f;
   constexpr int NE = BIG ? 4 : 1;  // hidden units per thread: H <= NE * threads
   float dh[NE], pu[NE], pr[NE], pc[NE], ph[NE], pg[NE];
@@ -305,7 +310,7 @@ void gru_bwd_kernel(const float *__restrict__ g, const float *__restrict__ act, 
         if (e < rows) gru_rows4(s, w + e, *reinterpret_cast<const float4 *>(vs + k0 + e));
         if (ll) gru_rows4(s, wl, *reinterpret_cast<const float4 *>(vs + k0 + RW + l));
       }
-      if (BIG) gru_stream(s, Wh, H, k0, RW + pl.lrows, rows, 2 * H, c, H, v4, vs);
+      if (BIG) gru_stream(s, Wh, H, k0, RW + pl.lrows, rows, 2 * H, c, H, vs);
       *reinterpret_cast<float4 *>(part + q * HC + 4 * c) = s;
     }
     lds_barrier();
@@ -378,8 +383,7 @@ static hipError_t gru_bwd_launch(GruPlan p, const float *g, const float *act, co
   static std::atomic<int> attr[kAttrDevices];
   const hipError_t e = ensure_lds_attr(reinterpret_cast<const void *>(gru_bwd_kernel<RW, BIG>), (int)p.lds, attr);
   if (e != hipSuccess) return e;
-  const int v4 = (H & 3) == 0 && (reinterpret_cast<uintptr_t>(Wh) & 15) == 0;
-  hipLaunchKernelGGL((gru_bwd_kernel<RW, BIG>), dim3(B), dim3(p.threads), p.lds, s, g, act, hprev, Wh, dG, T, H, seq, v4, p);
+  hipLaunchKernelGGL((gru_bwd_kernel<RW, BIG>), dim3(B), dim3(p.threads), p.lds, s, g, act, hprev, Wh, dG, T, H, seq, p);
   return hipGetLastError();
 }
 
