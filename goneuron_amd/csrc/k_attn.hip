@@ -1822,7 +1822,9 @@ constexpr int FA_NT = 256;
 // is about that low itself.  A workgroup with such a row (or one without a
 // finite sum) takes the tiles above the diagonal too.
 constexpr float FA_MASKED = -0.99e9f;
-__device__ __forceinline__ bool fa_whole(const float2 &ml) {  // (maximum, 1 / sum) of an ordinary row
+// (maximum, 1 / sum) of a row; the caller's workspace starts at any float
+typedef float fa_stat __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ bool fa_whole(const fa_stat &ml) {  // an ordinary row
   return ml.x > FA_MASKED && ml.y < __builtin_inff();
 }
 
@@ -2005,7 +2007,7 @@ __device__ __forceinline__ void fa_merge(fx4 (&o)[Fa<HD>::HX], float *buf) {
 template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                        const float *__restrict__ V, float *__restrict__ O,
-                                                       float2 *__restrict__ st, int T, int D, int NH, int hd,
+                                                       fa_stat *__restrict__ st, int T, int D, int NH, int hd,
                                                        int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B;
@@ -2128,7 +2130,7 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
 #pragma unroll
   for (int x = 0; x < F::HX; ++x) o[x] = o[x] * il;
   fa_store<HD, VEC>(O, o, base, qi, T, D, hd, lane);
-  if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = make_float2(m, il);
+  if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = fa_stat{m, il};
 }
 
 // c_i = gO_i . o_i (the lane's row) through the instructions, and in the order,
@@ -2165,7 +2167,7 @@ template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                          const float *__restrict__ V, const float *__restrict__ O,
                                                          const float *__restrict__ GO, float *__restrict__ GQ,
-                                                         const float2 *__restrict__ st, float *__restrict__ dr,
+                                                         const fa_stat *__restrict__ st, float *__restrict__ dr,
                                                          float *__restrict__ fl, int T, int D, int NH, int hd,
                                                          int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
@@ -2185,7 +2187,7 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_q_kernel(const float *__restrict
   fa_row<HD, VEC>(zb, GO + base, ri, T, D, hd, lane);
   float c = fa_rowdot<HD>(za, zb, lane);
   fa_row<HD, VEC>(za, Q + base, ri, T, D, hd, lane);
-  const float2 ml = ri < T ? st[(int64_t)pair * T + ri] : make_float2(0.f, 0.f);
+  const fa_stat ml = ri < T ? st[(int64_t)pair * T + ri] : fa_stat{0.f, 0.f};
   const int kend = causal ? min(T, rb * RB + RB) : T;
   float dsum = 0.f;  // of P (dP - c)
   auto row_sum = [&](float v) {  // over the lane groups and, with SP, the waves
@@ -2276,7 +2278,7 @@ template <int HD, bool SP, bool VEC>
 __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict__ Q, const float *__restrict__ K,
                                                          const float *__restrict__ V, const float *__restrict__ GO,
                                                          float *__restrict__ GK, float *__restrict__ GV,
-                                                         const float2 *__restrict__ st, const float *__restrict__ dr,
+                                                         const fa_stat *__restrict__ st, const float *__restrict__ dr,
                                                          const float *__restrict__ fl, int T, int D, int NH, int hd,
                                                          int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
@@ -2289,7 +2291,7 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
   const int64_t base = (int64_t)(pair / NH) * T * D + (pair % NH) * hd;
   const float is = 1.0f / (float)sqrt((double)hd);
   const int r0 = rb * RB + (SP ? 0 : 16 * w), ri = r0 + (lane & 15);  // the wave's and the lane's row
-  const float2 *stp = st + (int64_t)pair * T;
+  const fa_stat *stp = st + (int64_t)pair * T;
   const float *dp0 = dr + (int64_t)pair * T;
   float4 av[F::NL], bv[F::NL], za[F::HX], zb[F::HX];
   fx4 ga[F::HX], gb[F::HX];
@@ -2306,12 +2308,12 @@ __global__ __launch_bounds__(FA_NT) void fa_bwd_k_kernel(const float *__restrict
   }
   const int i0 = all ? 0 : rb * RB / F::KS * F::KS;  // first stage with a live query
   // the saved statistics and d of a stage's queries: wave w its tile w
-  float2 ml;
+  fa_stat ml;
   float dq;
   auto fetch_rows = [&](int k0) {
     const int t = k0 + 16 * w + lane;
     if (w >= KT || lane >= 16) return;
-    ml = t < T ? stp[t] : make_float2(0.f, 0.f);  // rows past the end: probability 0
+    ml = t < T ? stp[t] : fa_stat{0.f, 0.f};  // rows past the end: probability 0
     dq = t < T ? dp0[t] : 0.f;
   };
   fa_fetch<HD, SP, VEC>(av, Q + base, i0, T, D, hd);
@@ -2400,7 +2402,7 @@ static hipError_t fa_launch(const float *Q, const float *K, const float *V, floa
   const int hd = D / NH, rb = SP ? 16 : FA_B, nb = (T + rb - 1) / rb;
   const int64_t np = (int64_t)B * NH;
   if (np * nb * 2 > 0x7fffffff) return hipErrorInvalidValue;
-  float2 *st = reinterpret_cast<float2 *>(S);
+  fa_stat *st = reinterpret_cast<fa_stat *>(S);
   float *dr = S + 2 * np * T, *fl = S + 3 * np * T;
   const dim3 grid((unsigned)(np * nb)), block(FA_NT);
   if (!GO) {

@@ -15,17 +15,20 @@ from gpuutil import DBuf, TOL, log
 pytestmark = pytest.mark.gpu
 
 
-def _mha(dev, B, T, D, NH, causal, p, x, g):
+def _mha(dev, B, T, D, NH, causal, p, x, g, shift=0):
+    """shift: the workspace starts that many floats past its aligned start."""
     from goneuron_amd._lib import check, lib
     L = lib()
     ws = C.c_int64()
     check(None, L.gn_mha_workspace(B, T, D, NH, 0, C.byref(ws)))
     dx, dp, dg = DBuf(dev, x), DBuf(dev, p), DBuf(dev, g)
     dout, dgr, dgin, dwk = (DBuf(dev, np.full(s, np.nan, np.float32))
-                            for s in ((B, T * D), p.shape, (B, T * D), ws.value))
+                            for s in ((B, T * D), p.shape, (B, T * D), ws.value + shift))
+    whole, dwk.p = dwk.p, C.c_void_p(dwk.p.value + 4 * shift)
     check(dev.h, L.gn_mha_forward(dev.h, dx.p, dp.p, dout.p, dwk.p, B, T, D, NH, causal, 0))
     check(dev.h, L.gn_mha_backward(dev.h, dx.p, dp.p, dg.p, dgr.p, dgin.p, dwk.p, B, T, D, NH, causal, 0,
                                    C.c_float(np.float32(1) / np.float32(B))))
+    dwk.p = whole
     return dout.get(), dgr.get(), dgin.get()
 
 
@@ -180,3 +183,16 @@ def test_attn_masked_keys_with_weight(dev, oracle, T, D, NH, rows):
         a, b = (z[i * n1:i * n1 + D * D].reshape(D, D) for z in (got, gr))
         k = rows_ if i == 0 else slice(None)
         assert max_rel(a[k], b[k]) <= TOL, name
+
+
+@pytest.mark.parametrize("T,D,NH,causal,shift", [(150, 64, 2, 1, 1), (70, 96, 1, 0, 3), (200, 24, 1, 1, 2), (33, 48, 1, 0, 1)])
+def test_attn_workspace_at_any_float(dev, T, D, NH, causal, shift):
+    """A workspace that starts at any float gives what an aligned one gives (the
+    GEMMs around the attention sum in another order there)."""
+    log(f"attention T={T} D={D} heads={NH} workspace {shift} floats past its start")
+    rng = np.random.default_rng(T)
+    p = (rng.normal(size=4 * (D * D + D)) / np.sqrt(D)).astype(np.float32)
+    x, g = (rng.normal(size=(2, T * D)).astype(np.float32) for _ in range(2))
+    a, b = _mha(dev, 2, T, D, NH, causal, p, x, g), _mha(dev, 2, T, D, NH, causal, p, x, g, shift)
+    for u, v in zip(a, b):
+        assert np.isfinite(v).all() and max_rel(v, u) <= TOL
