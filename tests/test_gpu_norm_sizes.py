@@ -70,3 +70,10 @@ def test_norm_sizes(dev, kind, rows, N, shift):
         # a single column has x - mean = 0: the results are exact zeros or rounding
         r = np.abs(got - w.ravel()).max() / max(np.abs(w).max(), 1e-30) if np.abs(w).max() > 1e-6 else np.abs(got).max()
         assert r <= TOL, (name, r)
+
+
+@pytest.mark.parametrize("kind", ["ln", "rms"])
+@pytest.mark.parametrize("rows,N,shift", [(130, 63, 0), (5000, 64, 0), (130, 64, 3), (131, 65, 0), (129, 68, 0), (9, 2, 0)])
+def test_norm_short_rows(dev, kind, rows, N, shift):
+    """Both sides of the longest row that takes a column per lane."""
+    test_norm_sizes(dev, kind, rows, N, shift)
