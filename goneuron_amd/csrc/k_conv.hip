@@ -799,7 +799,9 @@ hipError_t launch_conv_fwd(const float *x, const float *w, const float *bias, fl
     }
   }
   if (pool_out) return hipErrorInvalidValue;
-  if (s.H >= 1 && s.W >= 1 && s.oH >= 1 && s.oW >= 1 && (int64_t)B * s.outC <= 65535 && s.outC >= 4) {
+  // the grid's y dimension: groups of eight channels (of four only where the
+  // whole grid of eights stays below 1024)
+  if (s.H >= 1 && s.W >= 1 && s.oH >= 1 && s.oW >= 1 && (int64_t)B * ((s.outC + 7) / 8) <= 65535 && s.outC >= 4) {
     if (s.k == 3 && s.stride == 1 && s.pad == 1) return conv_fwd_oc<3, true>(x, w, bias, out, s, B, fwd, st);
     if (s.k == 3) return conv_fwd_oc<3, false>(x, w, bias, out, s, B, fwd, st);
     if (s.k == 1) return conv_fwd_oc<1, false>(x, w, bias, out, s, B, fwd, st);

@@ -40,3 +40,39 @@ def test_conv_forward_sizes(dev, oracle, B, inC, HW, outC, k, s, p, act):
         np.testing.assert_array_equal(dout.get(), want[rows])
     else:
         assert np.abs(dout.get() - want[rows]).max() <= TOL * np.abs(want).max()
+
+
+def _conv64(x, w, b, k, s, p):
+    """Float64, with the reference's k3 s1 p1 rule: the first and last columns of
+    interior rows hold the bias alone."""
+    B, C, H, W = x.shape
+    oH, oW = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (p, p), (p, p)))
+    z = np.zeros((B, w.shape[0], oH, oW))
+    for i in range(k):
+        for j in range(k):
+            z += np.einsum("bchw,oc->bohw", xp[:, :, i:i + s * oH:s, j:j + s * oW:s][:, :, :oH, :oW], w[:, :, i, j].astype(np.float64))
+    if (k, s, p) == (3, 1, 1):
+        z[:, :, 1:oH - 1, 0] = 0
+        z[:, :, 1:oH - 1, oW - 1] = 0
+    return z + b[:, None, None]
+
+
+# planes higher than wide and wider than high; more than 65535 (sample, channel)
+# planes, which still are at most 65535 groups of eight, and more than that
+@pytest.mark.parametrize("B,inC,H,W,outC,k,s,p", [
+    (2, 5, 7, 19, 4, 3, 1, 1), (2, 6, 21, 3, 9, 3, 1, 1), (1, 7, 1, 40, 5, 3, 1, 1), (1, 7, 40, 1, 5, 3, 1, 1),
+    (2, 5, 9, 30, 7, 3, 2, 1), (2, 5, 30, 9, 8, 5, 1, 2), (2, 8, 17, 6, 12, 1, 1, 0), (1, 5, 6, 33, 6, 1, 2, 0),
+    (130, 5, 33, 12, 12, 3, 1, 1), (1100, 5, 4, 3, 64, 3, 1, 1), (9000, 1, 2, 3, 59, 1, 1, 0)])
+def test_conv_forward_planes(dev, B, inC, H, W, outC, k, s, p):
+    from goneuron_amd._lib import check, lib
+    L = lib()
+    log(f"conv2d forward B={B} inC={inC} {H}x{W} outC={outC} k={k} s={s} p={p}")
+    rng = np.random.default_rng(B + H * 7 + W)
+    x = rng.normal(size=(B, inC, H, W)).astype(np.float32)
+    w, b = (rng.normal(size=(outC, inC, k, k)) * 0.2).astype(np.float32), rng.normal(size=outC).astype(np.float32)
+    want = _conv64(x, w, b, k, s, p)
+    dx, dp = DBuf(dev, x), DBuf(dev, np.concatenate([w.ravel(), b]))
+    dout = DBuf(dev, np.full(want.shape, np.nan, np.float32))
+    check(dev.h, L.gn_conv2d_forward(dev.h, dx.p, dp.p, dout.p, B, inC, H, W, outC, k, s, p, 6))
+    assert np.abs(dout.get() - want).max() <= TOL * np.abs(want).max()
