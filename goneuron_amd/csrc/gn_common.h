@@ -553,6 +553,8 @@ hipError_t launch_ln_bwd_part(const float *g, const float *gpool, int poolT, con
                               const float *gam, const float *stats, float *dx, float *part, float *tsum,
                               int rows, int N, hipStream_t s, const float *tsx = nullptr,
                               float *tss = nullptr, int tsB = 0, int tsT = 0, int tsN = 0);
+// work may be null where norm_bwd_one_pass(N, ws_cap)
+bool norm_bwd_one_pass(int N, size_t ws_cap);
 hipError_t launch_ln_bwd(const float *g, const float *x, const float *gam, const float *stats, float *dx,
                          float *dgam, float *dbet, float *work, int rows, int N, float scale, float *ws,
                          size_t ws_cap, hipStream_t s);

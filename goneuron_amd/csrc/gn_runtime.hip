@@ -869,9 +869,10 @@ static int alloc_batch(gn_model *M) {
       if ((rc = model_balloc(M, 3 * rows * D, &t.GQ))) return rc;
       t.GK = t.GQ + rows * D;
       t.GV = t.GK + rows * D;
-      float **dbufs[] = {&t.O, &t.RES1, &t.N1, &t.RES2, &t.G1, &t.COMB, &t.G2, &t.GO, &t.GX};
+      float **dbufs[] = {&t.O, &t.RES1, &t.N1, &t.RES2, &t.G1, &t.COMB, &t.G2, &t.GO};
       for (float **b : dbufs)
         if ((rc = model_balloc(M, rows * D, b))) return rc;
+      if (!norm_bwd_one_pass(R.D, c->scratch_floats) && (rc = model_balloc(M, rows * D, &t.GX))) return rc;
       if ((rc = model_balloc(M, rows * FF, &t.MID))) return rc;
       if ((rc = model_balloc(M, rows * FF, &t.DZ1))) return rc;
       if ((rc = model_balloc(M, rows * 2, &t.st1))) return rc;
@@ -974,14 +975,18 @@ static int alloc_batch(gn_model *M) {
     }
     if (R.d.kind == GN_LAYER_RMSNORM) {
       if ((rc = model_balloc(M, (size_t)max_batch * (R.in_len / R.D), &R.rmsv))) return rc;
-      if ((rc = model_balloc(M, (size_t)max_batch * R.in_len, &R.gx))) return rc;
+      if (!norm_bwd_one_pass(R.D, c->scratch_floats) &&
+          (rc = model_balloc(M, (size_t)max_batch * R.in_len, &R.gx)))
+        return rc;
     }
     if (R.d.kind == GN_LAYER_LAYERNORM) {
-      // per-row (mean, std); g * xhat for the gamma sums when the one-pass
-      // backward does not fit the scratch; an input-gradient sink when the
-      // layer is first (the backward kernels always write dx)
+      // per-row (mean, std); g * xhat for the gamma sums of rows beyond the
+      // one-pass backward; an input-gradient sink when the layer is first (the
+      // backward kernels always write dx)
       if ((rc = model_balloc(M, (size_t)max_batch * (R.in_len / R.D) * 2, &R.rmsv))) return rc;
-      if ((rc = model_balloc(M, (size_t)max_batch * R.in_len, &R.gx))) return rc;
+      if (!norm_bwd_one_pass(R.D, c->scratch_floats) &&
+          (rc = model_balloc(M, (size_t)max_batch * R.in_len, &R.gx)))
+        return rc;
       if (i == 0 && (rc = model_balloc(M, (size_t)max_batch * R.in_len, &R.zbuf))) return rc;
     }
     if (R.d.kind == GN_LAYER_MHA) {

@@ -1754,13 +1754,17 @@ hipError_t launch_tb_params(TbParamSet &set, int B, float scale, hipStream_t s) 
   return hipGetLastError();
 }
 
-// rows longer than NB_MAXN: the row kernel writes g * xhat to work, column sums follow
+// the block partials of LayerNorm's two sums must fit the scratch
+bool norm_bwd_one_pass(int N, size_t ws_cap) { return N <= NB_MAXN && (size_t)NB_BLOCKS * 2 * N <= ws_cap; }
+
+// otherwise the row kernel writes g * xhat to work (rows x N), column sums follow
 hipError_t launch_ln_bwd(const float *g, const float *x, const float *gam, const float *stats, float *dx,
                          float *dgam, float *dbet, float *work, int rows, int N, float scale, float *ws,
                          size_t ws_cap, hipStream_t s) {
   if (rows <= 0) return hipSuccess;
-  if (N <= NB_MAXN && (size_t)NB_BLOCKS * 2 * N <= ws_cap)
+  if (norm_bwd_one_pass(N, ws_cap))
     return norm_bwd_rows<false>(g, x, gam, stats, dx, dgam, dbet, rows, N, scale, ws, s);
+  if (!work) return hipErrorInvalidValue;
   hipLaunchKernelGGL(ln_bwd_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, g, x, gam, stats, dx, work,
                      rows, N);
   const hipError_t e = hipGetLastError();
@@ -1794,8 +1798,9 @@ hipError_t launch_rms_bwd(const float *g, const float *x, const float *gam, cons
                           float *dgam, float *work, int rows, int N, float scale, float *ws, size_t ws_cap,
                           hipStream_t s) {
   if (rows <= 0) return hipSuccess;
-  if (N <= NB_MAXN && (size_t)NB_BLOCKS * N <= ws_cap)
+  if (norm_bwd_one_pass(N, ws_cap))
     return norm_bwd_rows<true>(g, x, gam, rms, dx, dgam, nullptr, rows, N, scale, ws, s);
+  if (!work) return hipErrorInvalidValue;
   hipLaunchKernelGGL(rms_bwd_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, g, x, gam, rms, dx, work,
                      rows, N);
   const hipError_t e = hipGetLastError();

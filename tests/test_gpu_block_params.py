@@ -43,7 +43,7 @@ def cases():
         "ln_rope": (dict(B=4, T=32, vocab=19, dim=32, heads=2, ff=32, rope=True), 2, True),
         # SwiGLU feed-forward (its ff1 gradient by GEMM), LayerNorm norms
         "ln_swiglu": (dict(B=4, T=16, vocab=31, dim=32, heads=2, ff=40, act="swiglu"), 1, True),
-        # 144 tokens: batched-GEMM attention, fused parameter launch
+        # 144 tokens: staged attention, fused parameter launch
         "ln_t144": (dict(B=3, T=144, vocab=17, dim=64, heads=2, ff=24), 1, True),
         # not fused: RMSNorm norms, and 20 tokens (16-row blocks span samples)
         "rms": (dict(B=5, T=32, vocab=37, dim=32, heads=4, ff=48, norm="rms"), 1, False),
@@ -65,7 +65,7 @@ def test_block_param_gradients(gn, oracle, dev, name):
     if fused:
         absent = set(UNFUSED)
         if kw.get("rope") or kw["T"] > 128:
-            # gQ, gK rotated after the attention backward, or the batched-GEMM
+            # gQ, gK rotated after the attention backward, or the staged
             # attention: the token sums of gQ, gK, gV by launch
             absent.discard("token_sum")
         assert FUSED <= names and not (absent & names), sorted(names)

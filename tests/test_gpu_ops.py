@@ -193,7 +193,7 @@ def test_layernorm_ops(dev, oracle, B, rows, N, eps):
 # ---------------------------------------------------------------- MultiHeadAttention
 @pytest.mark.parametrize("B,T,D,NH,causal,rope", [
     (4, 16, 64, 4, 1, 0), (3, 32, 64, 2, 0, 0), (2, 12, 48, 3, 1, 1), (5, 8, 32, 1, 0, 1),
-    # beyond the fused kernels (T > 128 or heads wider than 32): the batched-GEMM path
+    # beyond the fused kernels (T > 128 or heads wider than 32): the staged kernels
     (2, 136, 80, 2, 1, 0), (3, 40, 128, 2, 0, 1), (1, 200, 96, 3, 1, 1)])
 def test_mha_ops(dev, oracle, B, T, D, NH, causal, rope):
     L, check = _lib()
@@ -229,11 +229,12 @@ def test_mha_ops(dev, oracle, B, T, D, NH, causal, rope):
             _close(name + "." + part, got[sl], ref)
 
 
-@pytest.mark.parametrize("D,NH,T", [(128, 2, 2), (64, 2, 4)])
+@pytest.mark.parametrize("D,NH,T", [(128, 2, 2), (64, 2, 4), (260, 2, 2)])
 def test_mha_ops_beyond_grid_limit(dev, oracle, D, NH, T):
     """More (sample, head) pairs than a grid dimension holds (33,000 samples x
-    2 heads): the batched-GEMM path (heads 64 wide) runs the pairs in chunks,
-    the fused path (heads 32 wide) takes them on the grid's x dimension.  The
+    2 heads): the batched-GEMM path (heads 130 wide) runs the pairs in chunks,
+    the staged path (heads 64 wide) and the fused path (heads 32 wide) take
+    them on the grid's x dimension.  The
     batch repeats 10 distinct samples 3,300 times, so every output row equals
     its distinct sample's and the batch-averaged gradients equal the 10-sample
     batch's, which the oracle computes."""

@@ -631,7 +631,7 @@ def test_gpt_batch_over_64_samples(gn, oracle):
 def test_gpt_attention_shapes(gn, oracle, T, dim, heads, causal):
     """Odd sequence lengths and head dims (LDS zero padding), the non-causal
     path and a block-crossing causal mask, with a random block.  T > 128 or
-    heads wider than 32 (the last three) take the batched-GEMM attention
+    heads wider than 32 (the last three) take the staged attention
     (transformer.go:405-690 has no size limit)."""
     from goneuron_amd import configs
     cfg = configs.gpt(B=3, T=T, vocab=29, dim=dim, heads=heads, ff=24, causal=causal)
@@ -655,7 +655,7 @@ def test_gpt_block_ext(gn, oracle, act, norm, rope, causal, workers):
 
 def test_gpt_block_ext_long(gn, oracle):
     """SwiGLU, RMSNorm and RoPE over 160 tokens with 48-wide heads (the
-    batched-GEMM attention), causal, 2 steps with 2 workers."""
+    staged attention), causal, 2 steps with 2 workers."""
     from goneuron_amd import configs
     cfg = configs.gpt(B=4, T=160, vocab=31, dim=96, heads=2, ff=64, act="swiglu", norm="rms", rope=True)
     _compare_step(gn, oracle, cfg, steps=2, workers=2, perturb=_random_block(cfg, scale=0.1))

@@ -138,7 +138,7 @@ def cases():
                                    {"kind": "gap1d", "T": T, "dim": D},
                                    _dense(D, 4, "softmax", True)]),
                       (rng.integers(0, V, size=(B, T)).astype(np.float32), _onehot(rng, B, 4)))
-    # non-causal attention with heads wider than 32 (the batched-GEMM path), last
+    # non-causal attention with heads wider than 32 (the staged kernels), last
     out["mha_wide_out"] = (dict(num=35, name="mha_wide_out", B=B, loss="mse", lr=1e-3, x="normal",
                                 in_len=5 * 80,
                                 layers=[{"kind": "mha", "heads": 2, "T": 5, "causal": False, "dim": 80}]),
@@ -210,8 +210,8 @@ def test_layer_arrangements(gn, oracle, name):
 def test_transformer_batch_times_heads_beyond_grid(gn, oracle, dim):
     """A TransformerBlock training step over 8,200 samples x 8 heads (more
     (sample, head) pairs than a grid dimension holds): heads 2 wide take the
-    fused kernels (pairs on the grid's x dimension), heads 40 wide the
-    batched GEMMs in chunks of samples.  The batch repeats 10 distinct
+    fused kernels, heads 40 wide the staged ones (pairs on the grid's x
+    dimension both).  The batch repeats 10 distinct
     samples 820 times, so its loss and batch-averaged gradients equal the
     10-sample batch's, which the oracle computes; the last sample (the one
     the embedding gradient comes from, Q12) is the 10th distinct one."""
