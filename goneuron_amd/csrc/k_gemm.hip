@@ -745,7 +745,7 @@ template <int BKW, int NS, int RN, bool AK, bool BKC, int EPI>
 __global__ __launch_bounds__(NT4)
 __attribute__((amdgpu_waves_per_eu(NS * BKW * (128 + RN) <= 16384 ? 2 : 1,
                                    NS * BKW * (128 + RN) <= 16384 ? 2 : 1)))
-void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
+void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n) {
   constexpr int RM = 128, TM = 2, TN = RN / 64;
   constexpr int NLA = RM * BKW / 4 / NT4, NLB = RN * BKW / 4 / NT4;  // direct loads per thread
   constexpr int QN = BKW / 16;  // quarters of 8 MFMA steps per stage
@@ -763,9 +763,7 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
   const int half = lane >> 5, l32 = lane & 31;
   const int koff = half * (BKW / 2);
   const int M = p.M, N = p.N;
-  const int kbeg = blockIdx.y * kchunk;
-  const int kend = min(p.K, kbeg + kchunk);
-  const int nk = (kend - kbeg) / BKW;  // >= 1, full stages (checked by the launcher)
+  const int nk = p.K / BKW;  // >= 1, full stages (checked by the launcher)
   const int mrow = wm * (RM / 2), ncol = wn * (RN / 2);
 
   floatx16 acc[TM][TN];
@@ -778,7 +776,7 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
 
 #pragma unroll
   for (int st = 0; st < NS; ++st) {
-    const int k1 = kbeg + min(st, nk - 1) * BKW;
+    const int k1 = min(st, nk - 1) * BKW;
     load_tile_direct<RM, AK, NT4, BKW>(p.A, p.lda, M, m0, k1, As[st]);
     load_tile_direct<RN, BKC, NT4, BKW>(p.B, p.ldb, N, n0, k1, Bs[st]);
   }
@@ -839,7 +837,7 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n, int kchunk) {
     {
       // stage kt+NS into stage kt's buffer, which every wave finished
       // reading before this barrier
-      const int k2 = kbeg + min(kt + NS, nk - 1) * BKW;
+      const int k2 = min(kt + NS, nk - 1) * BKW;
       load_tile_direct<RM, AK, NT4, BKW>(p.A, p.lda, M, m0, k2, As[cur]);
       load_tile_direct<RN, BKC, NT4, BKW>(p.B, p.ldb, N, n0, k2, Bs[cur]);
     }
@@ -1221,9 +1219,9 @@ static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int 
       // its step; at K = 1024 the C3 step lost 3 %); else 64-deep stages, one
       // block per CU.
       if (tm * tn >= 512 || kchunk <= 256)
-        hipLaunchKernelGGL((gemm_f32_mfma_w4<32, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn, kchunk);
+        hipLaunchKernelGGL((gemm_f32_mfma_w4<32, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn);
       else
-        hipLaunchKernelGGL((gemm_f32_mfma_w4<64, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn, kchunk);
+        hipLaunchKernelGGL((gemm_f32_mfma_w4<64, 2, 128, AK, BKC, EPI>), grid, dim3(NT4), 0, s, a, tm, tn);
       return hipGetLastError();
     }
   } else {
@@ -1245,12 +1243,21 @@ template <int R, int EPI>
 static hipError_t launch_e(char ta, char tb, bool vec, bool ktail, const GemmArgs &a, int tm, int tn,
                            int splits, int kchunk, hipStream_t s) {
   // op(A) 'N' -> A is M x K, K contiguous.  op(B) 'T' -> B is N x K, K contiguous.
+  // Orders that callers use: forward products with a bias NT, their residuals NT
+  // and the backward's NN, dX with an activation derivative NN; plain products
+  // and partial sums all four.
+  constexpr bool plain = EPI == EPI_SCALE || EPI == EPI_PARTIAL;
   const bool ak = (ta == 'N');
   const bool bk = (tb == 'T');
-  if (ak && bk) return launch_t<R, true, true, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
-  if (ak && !bk) return launch_t<R, true, false, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
-  if (!ak && bk) return launch_t<R, false, true, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
-  return launch_t<R, false, false, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
+  if constexpr (EPI != EPI_DACT)
+    if (ak && bk) return launch_t<R, true, true, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
+  if constexpr (EPI != EPI_BIAS_ACT)
+    if (ak && !bk) return launch_t<R, true, false, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
+  if constexpr (plain) {
+    if (!ak && bk) return launch_t<R, false, true, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
+    if (!ak && !bk) return launch_t<R, false, false, EPI>(vec, ktail, a, tm, tn, splits, kchunk, s);
+  }
+  return hipErrorNotSupported;
 }
 
 template <int R>
