@@ -2137,9 +2137,13 @@ __global__ __launch_bounds__(FA_NT) void fa_fwd_kernel(const float *__restrict__
     l = ((wl[0][i] + wl[1][i]) + wl[2][i]) + wl[3][i];
     if (w > 0) return;
   }
+  // divided, not multiplied by 1 / l: one rounding, where the reciprocal's would
+  // be common to the whole row
   const float il = 1.0f / l;
 #pragma unroll
-  for (int x = 0; x < F::HX; ++x) o[x] = o[x] * il;
+  for (int x = 0; x < F::HX; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[x][r] = o[x][r] / l;
   fa_store<HD, VEC>(O, o, base, qi, T, D, hd, lane);
   if (lane < 16 && qi < T) st[(int64_t)pair * T + qi] = fa_stat{m, il};
 }
