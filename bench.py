@@ -30,6 +30,8 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense fp32 matrix (and vector) peak
 PEAK_FP64_MFMA_TFLOPS = 78.6
+# large backward GEMMs run as six bf16 partial products per fp32 product
+PEAK_SPLIT_TFLOPS = 2500.0 / 6
 PEAK_HBM_GBPS = 8000.0
 # the CPU share of one GPU on the GPU boxes (their nproc shows the whole host)
 CPU_SHARE = 16
@@ -61,6 +63,8 @@ def gemm_traffic_per_launch():
 
 def kernel_bound(name):
     """(bound, peak, unit) a kernel is judged against."""
+    if name.startswith("gemm_") and name.endswith("_split"):
+        return "mfma_bf16x6", PEAK_SPLIT_TFLOPS, "TFLOP/s"
     if name.startswith("gemm_") or name in ("attn_fwd", "attn_bwd", "conv_wgrad", "conv_dgrad"):
         return "mfma", PEAK_FP32_MFMA_TFLOPS, "TFLOP/s"
     if name == "lstm_gram":
@@ -303,13 +307,16 @@ def run_config(name, args, dev, with_cpu, cpu_budget, threads):
     g_ms = sum(v["ms_per_step"] for v in gemm.values()) * K
     g_n = sum(v["launches_per_step"] for v in gemm.values()) * K
     g_units = sum(v["units_per_launch"] * v["launches_per_step"] for v in gemm.values()) * K
+    # each product at the peak of the matrix cores that run it
+    g_floor = sum(v["units_per_launch"] * v["launches_per_step"] / v["peak"] for v in gemm.values()) * K
     res = {
         "workload": name, "batch": B, "workers": workers, "params": nparams,
         "value": B * K / elapsed, "unit": "samples/s", "ms_per_step": elapsed * 1e3 / K,
         "instrumented_ms_per_step": elapsed_ev * 1e3 / K,
         "kernels_per_step": sum(v["launches_per_step"] for v in kernels.values()),
         "gemm": {"launches_per_step": g_n / K, "ms_per_step": g_ms / K,
-                 "flops_per_step": g_units / K,
+                 "flops_per_step": g_units / K, "peak_tflops": g_units / g_floor if g_floor > 0 else None,
+                 "kernels": sorted(gemm),
                  "achieved_tflops": g_units / (g_ms * 1e-3) / 1e12 if g_ms > 0 else None,
                  "avg_launch_ms": g_ms / g_n if g_n else None},
         "dominant": dominant(kernels),
@@ -461,11 +468,14 @@ def final_line(args, cfg, head, others, host, traffic):
     per other configuration.  Full per-kernel tables go to DETAIL_PATH."""
     g = head["gemm"]
     if g["launches_per_step"] and g["achieved_tflops"]:
-        # GEMM family of the step: every launch of the fp32 MFMA GEMM kernels
-        roof = {"bound": "mfma", "achieved": _r(g["achieved_tflops"]), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": _r(g["achieved_tflops"] / PEAK_FP32_MFMA_TFLOPS),
+        # GEMM family of the step: launches on the fp32 matrix cores and, named
+        # *_split, on the bf16 ones (six partial products each); the peak is the
+        # rate at which both together would run at theirs
+        peak = g.get("peak_tflops") or PEAK_FP32_MFMA_TFLOPS
+        roof = {"bound": "mfma", "achieved": _r(g["achieved_tflops"]), "peak": _r(peak),
+                "unit": "TFLOP/s", "frac": _r(g["achieved_tflops"] / peak),
                 "traffic": traffic,
-                "kernel": "gemm_f32_mfma (gemm_fwd, gemm_dx, gemm_dw)",
+                "kernel": "GEMMs (" + ", ".join(g.get("kernels") or ["gemm_fwd", "gemm_dx", "gemm_dw"]) + ")",
                 "flops_per_launch": _r(g["flops_per_step"] / g["launches_per_step"]),
                 "avg_launch_ms": _r(g["avg_launch_ms"]),
                 "launches_per_step": g["launches_per_step"]}

@@ -134,6 +134,9 @@ enum GemmEpi : int { EPI_SCALE = 0, EPI_BIAS_ACT = 1, EPI_DACT = 2, EPI_BIAS_ADD
 // op(A) layout: 'N' = A[m*lda+k] (K contiguous), 'T' = A[k*lda+m].
 // op(B) layout: 'N' = B[k*ldb+n] (N contiguous), 'T' = B[n*ldb+k].
 hipError_t launch_gemm(char ta, char tb, int epi, const GemmArgs &a, hipStream_t s);
+// launch_gemm runs this (unbatched) product on the bf16 matrix cores, as six
+// partial products of its operands' three-way split
+bool gemm_on_split(char ta, char tb, int epi, const GemmArgs &a);
 
 hipError_t launch_adam(float *p, const float *g, float *m, float *v, int64_t n, float efflr,
                        float b1, float b2, float omb1, float omb2, float eps, hipStream_t s,

@@ -344,7 +344,7 @@ hipError_t dense_bwd_core(gn_ctx *c, const float *x, const float *W, const float
   a.alpha = scale;
   a.ws = wscr; a.ws_cap = wcap;
   if (!skip_dw) {
-    KTimer kt(c, GN_KCLASS_GEMM, "gemm_dw", gemm_flops(a), ws);
+    KTimer kt(c, GN_KCLASS_GEMM, gemm_on_split('T', 'N', EPI_SCALE, a) ? "gemm_dw_split" : "gemm_dw", gemm_flops(a), ws);
     e = launch_gemm('T', 'N', EPI_SCALE, a, ws);
     if (e != hipSuccess) return e;
   }
@@ -362,13 +362,12 @@ hipError_t dense_bwd_core(gn_ctx *c, const float *x, const float *W, const float
       d.cs_done = &cs_done;
     }
     {
-      KTimer kt(c, GN_KCLASS_GEMM, "gemm_dx", gemm_flops(d));
+      const int epi = gin_aux ? EPI_DACT : EPI_SCALE;
+      KTimer kt(c, GN_KCLASS_GEMM, gemm_on_split('N', 'N', epi, d) ? "gemm_dx_split" : "gemm_dx", gemm_flops(d));
       if (gin_aux) {
         d.aux = gin_aux; d.ldaux = in; d.act = gin_deriv; d.colscale = gin_colscale;
-        e = launch_gemm('N', 'N', EPI_DACT, d, c->stream);
-      } else {
-        e = launch_gemm('N', 'N', EPI_SCALE, d, c->stream);
       }
+      e = launch_gemm('N', 'N', epi, d, c->stream);
     }
     if (e != hipSuccess) return e;
     if (cs_in_dx && !cs_done) {
@@ -1593,7 +1592,7 @@ static hipError_t gemm_nn(gn_ctx *c, const float *A, const float *Wm, float *C, 
   a.C = C; a.ldc = N; a.alpha = 1.f; a.act = act;
   a.aux = aux; a.ldaux = N; a.aux_div = aux_div;
   a.ws = c->scratch; a.ws_cap = c->scratch_floats;
-  KTimer kt(c, GN_KCLASS_GEMM, "gemm_dx", gemm_flops(a));
+  KTimer kt(c, GN_KCLASS_GEMM, gemm_on_split('N', 'N', epi, a) ? "gemm_dx_split" : "gemm_dx", gemm_flops(a));
   return launch_gemm('N', 'N', epi, a, c->stream);
 }
 

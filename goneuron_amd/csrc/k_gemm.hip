@@ -1186,6 +1186,8 @@ __global__ __launch_bounds__(NT) void gemm_splitk_reduce_wave(GemmArgs p, int sp
   }
 }
 
+static bool split_rule(int epi, bool vec, const GemmArgs &a);
+
 template <int R, bool AK, bool BKC, int EPI>
 static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int tn, int splits,
                           int kchunk, hipStream_t s) {
@@ -1202,14 +1204,10 @@ static hipError_t launch_t(bool vec, bool ktail, const GemmArgs &a, int tm, int 
     // residuals, the transformer's dX sums) stays on fp32 MFMAs too.  64-wide
     // tiles stay with eight waves of fp32 MFMAs, mostly faster there
     // (4096 x 256 x 1024 22 against 28 us).
-    // From five K stages on: four or fewer are bound by the operands' and C's
-    // traffic, and there the split only adds work (1664 x 1664 x 64 TN 10.3
-    // -> 11.3 us, 4096 x 4096 x 128 NT 54.5 -> 57.5; at K = 512 16384 x 512 x
-    // 512 is 73 -> 55).
     constexpr bool split = EPI == EPI_SCALE || EPI == EPI_DACT;
     if (vec && !ktail) {
       if constexpr (split)
-        if (!a.fwd && a.K > 4 * BK) {
+        if (split_rule(EPI, vec, a)) {
           hipLaunchKernelGGL((gemm_split_bf16<AK, BKC, EPI>), grid, dim3(SB_NT), 0, s, a, tm, tn);
           return hipGetLastError();
         }
@@ -1293,6 +1291,27 @@ bool gemm_segments_ok(const GemmArgs &a) {
   return a.kseg > 0 && a.kseg % BK == 0 && a.nbatch <= 1 && !a.defer_splits && !a.drop_out && !plan_big(a);
 }
 
+// float4 staging needs 16 B aligned rows and the contiguous extent % 4 == 0
+static bool gemm_vec(char ta, char tb, const GemmArgs &a) {
+  bool vec = aligned16(a.A) && aligned16(a.B) && (a.lda % 4 == 0) && (a.ldb % 4 == 0) &&
+             ((a.seg_A | a.seg_B) & 3) == 0;
+  vec = vec && (ta == 'N' ? a.K % 4 == 0 : a.M % 4 == 0);
+  vec = vec && (tb == 'T' ? a.K % 4 == 0 : a.N % 4 == 0);
+  return vec && a.K > 0;  // the pipelined loop assumes at least one K stage
+}
+
+// From five K stages on: four or fewer are bound by the operands' and C's
+// traffic, and there the split only adds work (1664 x 1664 x 64 TN 10.3 ->
+// 11.3 us, 4096 x 4096 x 128 NT 54.5 -> 57.5; at K = 512 16384 x 512 x 512 is 73
+// -> 55).
+static bool split_rule(int epi, bool vec, const GemmArgs &a) {
+  return (epi == EPI_SCALE || epi == EPI_DACT) && !a.fwd && vec && a.K % BK == 0 && a.K > 4 * BK;
+}
+
+bool gemm_on_split(char ta, char tb, int epi, const GemmArgs &a) {
+  return a.nbatch <= 1 && a.kseg <= 0 && plan_big(a) && split_rule(epi, gemm_vec(ta, tb, a), a);
+}
+
 hipError_t launch_gemm(char ta, char tb, int epi, const GemmArgs &a0, hipStream_t s) {
   if (a0.M <= 0 || a0.N <= 0) return hipSuccess;
   GemmArgs a = a0;
@@ -1305,13 +1324,7 @@ hipError_t launch_gemm(char ta, char tb, int epi, const GemmArgs &a0, hipStream_
     a.kseg = 0;
   }
   if (a.drop_out && (epi != EPI_BIAS_ACT || a.nbatch > 1 || !a.drop_mask)) return hipErrorInvalidValue;
-  // float4 staging needs 16 B aligned rows and the contiguous extent % 4 == 0
-  const bool ak = (ta == 'N'), bk = (tb == 'T');
-  bool vec = aligned16(a.A) && aligned16(a.B) && (a.lda % 4 == 0) && (a.ldb % 4 == 0) &&
-             ((a.seg_A | a.seg_B) & 3) == 0;
-  vec = vec && (ak ? (a.K % 4 == 0) : (a.M % 4 == 0));
-  vec = vec && (bk ? (a.K % 4 == 0) : (a.N % 4 == 0));
-  vec = vec && a.K > 0;  // the pipelined loop assumes at least one K stage
+  const bool vec = gemm_vec(ta, tb, a);
   // 128-wide tiles when they fill the 256 CUs, else 64-wide tiles; when even
   // those cannot fill the chip and K has at least 8 stages, split K (down to
   // one K stage per split: a lone tile runs at 1/256 of the chip).  Partials

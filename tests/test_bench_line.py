@@ -78,3 +78,16 @@ def test_kernel_floor_is_the_longer_of_launch_and_work():
     k2 = {"x": {"unit": "GB/s", "peak": 8000.0, "units_per_launch": 1.0, "us_per_launch": 5.0}}
     bench.add_floors(k2, None)
     assert "floor_us" not in k2["x"]
+
+
+def test_split_gemms_are_read_against_their_own_cores():
+    """*_split launches: a sixth of the bf16 peak; the family's peak is the rate
+    of both kinds at theirs."""
+    assert bench.kernel_bound("gemm_dw_split")[1] == bench.PEAK_SPLIT_TFLOPS
+    assert bench.kernel_bound("gemm_dw")[1] == bench.PEAK_FP32_MFMA_TFLOPS
+    args = argparse.Namespace(steps=20, warmup=5, config="wide")
+    head = fake_result("wide")
+    head["gemm"].update(peak_tflops=240.0, kernels=["gemm_dw_split", "gemm_fwd"])
+    roof = bench.final_line(args, {"name": "wide", "loss": "ce"}, head, {}, {}, None)["roofline"]
+    assert roof["peak"] == 240.0 and abs(roof["frac"] - 123.9123456 / 240) < 1e-3
+    assert "gemm_dw_split" in roof["kernel"]
