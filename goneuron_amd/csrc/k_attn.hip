@@ -1822,10 +1822,14 @@ bool attn_supported(int T, int D, int NH) {
 // The materialised form (batched GEMMs over the pairs, below) took a launch
 // per (sample, head) pair when T is odd, and otherwise moved 2 T^2 floats per
 // pair through HBM seven times.  The whole layer, forward + backward: B 8, T
-// 197, 3 heads of 64 1207 -> 106 us; B 4, T 512, 8 heads of 64, causal 310 ->
-// 216; a GPT step at B 16, T 256, 8 heads of 32 510 -> 319.  What bounds them
-// is the matrix pipe (forward 17 of 27 kilocycles at B 4, T 512, backward 62)
-// and, beside it, the vector work of the exponentials and the staging.
+// 197, 3 heads of 64 1204 -> 112 us; B 4, T 512, 8 heads of 64, causal 318 ->
+// 224; a GPT step at B 16, T 256, 8 heads of 32 484 -> 322; heads of 128 keep its
+// time at even T (B 4, T 512, 8 heads 598 -> 600, B 1, T 1024 450 -> 420).  Every
+// stage sums on its own before it is added: one chain of fp32 MFMAs over all
+// keys had 1.4 times the materialised form's error at T 486, now 0.75.  What
+// bounds them is the matrix pipe (B 4, T 512: 30 us forward, 40 + 44 backward,
+// 7 and 24 at the fp32 peak) and, beside it, the float64 exponentials and the
+// staging.
 // ---------------------------------------------------------------------------
 constexpr int FA_B = 64;    // rows per workgroup (16 per wave) where they fill the chip
 constexpr int FA_NT = 256;

@@ -39,9 +39,10 @@ namespace gn {
 // rows; the shares' partial sums meet in LDS.  What bounds a step then is the
 // 3H^2 (forward) or 2H^2 (backward) fused multiply-adds on one CU's vector
 // lanes (1.3 and 0.9 us at H = 256), the barriers between its phases and the
-// float64 activations: 3.7 us per forward and 2.3 us per backward step at
-// B = 64, H = 256 (the whole layer, T = 100: 3,962 -> 689 us; H = 64: 1,035 ->
-// 354, H = 320: 5,052 -> 1,805).
+// float64 activations: 3.7 us per forward and 2.0 us per backward step at
+// B = 64, H = 256 (the whole layer, T = 100: 3,957 -> 663 us; at T = 30 H = 64,
+// B = 300: 374 -> 166, H = 320, B = 128: 1,600 -> 572, H = 1024: 10,390 ->
+// 5,199).
 // Rows past the matrix hold zero weights and meet zero inputs.
 constexpr int GR_NT = 512;   // threads at most
 

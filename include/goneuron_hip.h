@@ -517,10 +517,12 @@ int gn_moe_backward(gn_ctx *ctx, const float *x, const float *params, const floa
                     float *gin, float *work, int32_t B, int32_t I, int32_t O, int32_t E, int32_t K,
                     int32_t training, float scale);
 
-/* Generic fp32 MFMA GEMM: C[M,N] = alpha * op(A) op(B); trans flags as BLAS
+/* Generic fp32 GEMM: C[M,N] = alpha * op(A) op(B); trans flags as BLAS
  * (A is M x K row-major when transA == 0, K x M when 1; B is K x N when
- * transB == 0, N x K when 1).  Stands in for matMulMPSPersistent
- * (metal_ops.m:1220-1233). */
+ * transB == 0, N x K when 1).  On fp32 MFMA; large ones with K a multiple of
+ * 64 from 320 on as six bf16 MFMA products of the operands' exact three-way
+ * split, with a smaller error over all of float32's range.  Stands in for
+ * matMulMPSPersistent (metal_ops.m:1220-1233). */
 int gn_gemm(gn_ctx *ctx, int32_t transA, int32_t transB, int32_t M, int32_t N, int32_t K,
             float alpha, const float *A, int32_t lda, const float *B, int32_t ldb, float *C,
             int32_t ldc);
