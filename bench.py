@@ -407,7 +407,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py runs on one GPU only (asked for --gpus {args.gpus}); the data-parallel "
-              "sharding across GPUs is a design (DESIGN.md), not built here.", file=sys.stderr)
+              "sharding across GPUs is a design, not built here.", file=sys.stderr)
         sys.exit(2)
     if args.calibrate_copy:
         calibrate_copy(args.calibrate_copy)

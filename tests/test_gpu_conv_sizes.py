@@ -76,3 +76,35 @@ def test_conv_forward_planes(dev, B, inC, H, W, outC, k, s, p):
     dout = DBuf(dev, np.full(want.shape, np.nan, np.float32))
     check(dev.h, L.gn_conv2d_forward(dev.h, dx.p, dp.p, dout.p, B, inC, H, W, outC, k, s, p, 6))
     assert np.abs(dout.get() - want).max() <= TOL * np.abs(want).max()
+
+
+@pytest.mark.parametrize("B,inC,outC", [(6000, 32, 8), (1500, 57, 4), (70, 64, 16)])
+def test_conv_weight_gradient_block_sums(dev, B, inC, outC):
+    """The blocks' partials of many slots: one block per sample here, whose
+    partial is one exact product (a single output gradient, inputs that are
+    powers of two), so what is left is the rounding of their sum.  It must not
+    exceed that of a wave per slot (64 chains, then a tree), restated in numpy;
+    a tenth is allowed for the draw."""
+    from goneuron_amd._lib import check, lib
+    L = lib()
+    log(f"conv2d weight gradient B={B} {inC} -> {outC} channels of 3x3")
+    rng = np.random.default_rng(B)
+    x = np.broadcast_to(np.exp2(rng.integers(-1, 2, size=(B, inC, 1, 1))), (B, inC, 3, 3)).astype(np.float32)
+    g = np.zeros((B, outC, 3, 3), np.float32)
+    g[:, :, 1, 1] = rng.uniform(1, 2, size=(B, outC))
+    n = outC * inC * 9
+    dx, dg = DBuf(dev, np.ascontiguousarray(x)), DBuf(dev, g)
+    dp, dout, dgr = (DBuf(dev, np.zeros(k, np.float32)) for k in (n + outC, g.shape, n + outC))
+    check(dev.h, L.gn_conv2d_backward(dev.h, dx.p, dp.p, dout.p, dg.p, dgr.p, None, B, inC, 3, 3, outC, 3, 1, 1, 6, 1.0))
+    got = dgr.get()[:n].reshape(outC, inC, 9)
+    terms = g[:, :, None, 1, 1] * x[:, None, :, 0, 0]  # exact
+    ref = terms.astype(np.float64).sum(0)
+    assert np.array_equal(got, np.broadcast_to(got[:, :, :1], got.shape))  # every tap meets the same products
+    lanes = [np.zeros((outC, inC), np.float32) for _ in range(64)]
+    for b in range(B):
+        lanes[b % 64] = lanes[b % 64] + terms[b]
+    while len(lanes) > 1:
+        lanes = [a + b for a, b in zip(lanes[:len(lanes) // 2], lanes[len(lanes) // 2:])]
+    rms = [np.sqrt(np.mean((v / ref - 1) ** 2)) for v in (got[:, :, 0], lanes[0])]
+    log(f"  rounding {rms[0]:.2e}, a wave per slot {rms[1]:.2e}")
+    assert rms[0] <= 1.1 * rms[1]
