@@ -801,7 +801,16 @@ hipError_t launch_conv_fwd(const float *x, const float *w, const float *bias, fl
   if (pool_out) return hipErrorInvalidValue;
   // the grid's y dimension: groups of eight channels (of four only where the
   // whole grid of eights stays below 1024)
-  if (s.H >= 1 && s.W >= 1 && s.oH >= 1 && s.oW >= 1 && (int64_t)B * ((s.outC + 7) / 8) <= 65535 && s.outC >= 4) {
+  // A thread evaluates its channels' activations one after the other.  Where that
+  // is the float64 tanh, the windows short and the grid small, it costs more than
+  // windows read once save, and a channel per thread is faster (B 16, 8 -> 12
+  // channels, 10 x 10 10.3 against 11.7 us, 48 workgroups of four channels; B 32, 5
+  // -> 8, 20 x 20 7.7 against 8.1, 128; beyond either limit B 8, 7 -> 9, 40 x 40 9.8
+  // against 9.3, 168; B 24, 10 -> 16, 16 x 16 13.0 against 11.4, 90 taps).
+  const int64_t wg4 = (int64_t)((s.oH * s.oW + CT - 1) / CT) * B * ((s.outC + 3) / 4);
+  const bool serial = fwd == F_TANH && s.inC * s.k * s.k <= 72 && wg4 <= 128;
+  if (s.H >= 1 && s.W >= 1 && s.oH >= 1 && s.oW >= 1 && (int64_t)B * ((s.outC + 7) / 8) <= 65535 && s.outC >= 4 &&
+      !serial) {
     if (s.k == 3 && s.stride == 1 && s.pad == 1) return conv_fwd_oc<3, true>(x, w, bias, out, s, B, fwd, st);
     if (s.k == 3) return conv_fwd_oc<3, false>(x, w, bias, out, s, B, fwd, st);
     if (s.k == 1) return conv_fwd_oc<1, false>(x, w, bias, out, s, B, fwd, st);

@@ -108,3 +108,10 @@ def test_conv_weight_gradient_block_sums(dev, B, inC, outC):
     rms = [np.sqrt(np.mean((v / ref - 1) ** 2)) for v in (got[:, :, 0], lanes[0])]
     log(f"  rounding {rms[0]:.2e}, a wave per slot {rms[1]:.2e}")
     assert rms[0] <= 1.1 * rms[1]
+
+
+@pytest.mark.parametrize("B,inC,HW,outC,k,s,p", [
+    (32, 5, 20, 8, 3, 1, 1), (33, 5, 20, 8, 3, 1, 1), (4, 8, 10, 12, 3, 1, 1), (4, 9, 10, 12, 3, 1, 1), (4, 2, 9, 7, 3, 2, 1)])
+def test_conv_forward_tanh(dev, oracle, B, inC, HW, outC, k, s, p):
+    """Both sides of the grid and window up to which tanh takes a channel per thread."""
+    test_conv_forward_sizes(dev, oracle, B, inC, HW, outC, k, s, p, 3)
