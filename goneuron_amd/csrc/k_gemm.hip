@@ -868,10 +868,11 @@ void gemm_f32_mfma_w4(GemmArgs p, int tiles_m, int tiles_n) {
 // 8 significant bits, round to nearest), and a product is the six partial
 // products down to 2^-16 of it (h h, h m, m h, m m, h l, l h; what is left out
 // is below 2^-26), by v_mfma_f32_32x32x16_bf16.  bf16 has float32's exponents,
-// so the parts of an unscaled value below 2^-110 would underflow (relative
-// error 1e-6 at 2^-114, 2e-3 at 2^-125): both operands are split times 2^24,
-// which makes every part of every float32, denormals too, zero or a normal
-// bf16, and the sums are multiplied by 2^-48 at the end.  These MFMAs run at 12 times the fp32 rate (1712
+// so the lower parts of an unscaled value below 2^-110 would underflow, and all
+// of a denormal (relative errors of up to 0.3 measured where the fp32 MFMA has
+// 3e-7): both operands are split times 2^24, which makes every part of every
+// float32, denormals too, zero or a normal bf16, and the sums are multiplied by
+// 2^-48 at the end (7e-8 then).  These MFMAs run at 12 times the fp32 rate (1712
 // against 142 TFLOP/s measured from registers), so six of them per product
 // leave a ceiling of 285 TFLOP/s.
 //
