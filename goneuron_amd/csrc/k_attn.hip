@@ -1815,7 +1815,8 @@ bool attn_supported(int T, int D, int NH) {
 // ---------------------------------------------------------------------------
 // Attention of any sequence length with heads of up to 128 (what the kernels
 // above do not hold in LDS at once), on fp32 MFMA 16x16x4 with their operand
-// layouts.  Nothing of size T x T is written: the forward keeps a running row maximum and sum over stages of keys and leaves
+// layouts.  Nothing of size T x T is written: the forward keeps a running row
+// maximum and sum over stages of keys and leaves
 // (maximum, 1 / sum) per row for the backward, which recomputes the
 // probabilities.  A workgroup is four waves that share the staged rows of the
 // other side in LDS.
@@ -2025,10 +2026,10 @@ __device__ __forceinline__ void fa_merge(fx4 (&o)[Fa<HD>::HX], float *buf) {
 // other side (their results meet in LDS), which gives a short batch four times
 // the workgroups; otherwise each wave has 16 rows of its own.
 template <int HD, bool SP, bool VEC>
-__global__ __launch_bounds__(FA_NT, fa_waves(HD, true)) void fa_fwd_kernel(const float *__restrict__ Q, const float *__restrict__ K,
-                                                       const float *__restrict__ V, float *__restrict__ O,
-                                                       fa_stat *__restrict__ st, int T, int D, int NH, int hd,
-                                                       int causal, int npair, int nb) {
+__global__ __launch_bounds__(FA_NT, fa_waves(HD, true))
+void fa_fwd_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
+                   float *__restrict__ O, fa_stat *__restrict__ st, int T, int D, int NH, int hd, int causal,
+                   int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
@@ -2188,12 +2189,11 @@ __device__ __forceinline__ float fa_rowdot(const float4 (&o)[Fa<HD>::HX], const 
 // few probabilities average that rounding, has the sum before its gQ and takes
 // it there too.
 template <int HD, bool SP, bool VEC>
-__global__ __launch_bounds__(FA_NT, fa_waves(HD, false)) void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K,
-                                                         const float *__restrict__ V, const float *__restrict__ O,
-                                                         const float *__restrict__ GO, float *__restrict__ GQ,
-                                                         const fa_stat *__restrict__ st, float *__restrict__ dr,
-                                                         float *__restrict__ fl, int T, int D, int NH, int hd,
-                                                         int causal, int npair, int nb) {
+__global__ __launch_bounds__(FA_NT, fa_waves(HD, false))
+void fa_bwd_q_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
+                     const float *__restrict__ O, const float *__restrict__ GO, float *__restrict__ GQ,
+                     const fa_stat *__restrict__ st, float *__restrict__ dr, float *__restrict__ fl, int T, int D,
+                     int NH, int hd, int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
@@ -2299,12 +2299,11 @@ __global__ __launch_bounds__(FA_NT, fa_waves(HD, false)) void fa_bwd_q_kernel(co
 
 // Key blocks: gK and gV over the live queries, four products per tile pair.
 template <int HD, bool SP, bool VEC>
-__global__ __launch_bounds__(FA_NT, fa_waves(HD, false)) void fa_bwd_k_kernel(const float *__restrict__ Q, const float *__restrict__ K,
-                                                         const float *__restrict__ V, const float *__restrict__ GO,
-                                                         float *__restrict__ GK, float *__restrict__ GV,
-                                                         const fa_stat *__restrict__ st, const float *__restrict__ dr,
-                                                         const float *__restrict__ fl, int T, int D, int NH, int hd,
-                                                         int causal, int npair, int nb) {
+__global__ __launch_bounds__(FA_NT, fa_waves(HD, false))
+void fa_bwd_k_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
+                     const float *__restrict__ GO, float *__restrict__ GK, float *__restrict__ GV,
+                     const fa_stat *__restrict__ st, const float *__restrict__ dr, const float *__restrict__ fl,
+                     int T, int D, int NH, int hd, int causal, int npair, int nb) {
   using F = Fa<HD, SP>;
   constexpr int RB = SP ? 16 : FA_B, KT = F::KS / 16;
   __shared__ __align__(16) float sh[2 * F::KS * F::P];
